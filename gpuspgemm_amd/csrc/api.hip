@@ -472,6 +472,9 @@ struct Context {
     // array instead of summing the earlier tiles per workgroup (quadratic
     // in the tile count); SPG_TILE_PREFIX_MIN overrides it
     int tile_prefix_min = kTilePrefixMin;
+    // entries of B from which the kernels take 64-bit byte offsets into its
+    // arrays (8 bytes a value pass 4 GiB there); SPG_WIDE_MIN overrides it
+    int wide_min = 1 << 29;
     Lane lane;  // graph replay and profiling run here, one call at a time
     Lane noalloc_lane;             // spg_multiply_noalloc, one call at a time
     char* noalloc_base = nullptr;  // this device's address of `scratch`
@@ -603,6 +606,7 @@ spg_status ensure_context(Context*& out) {
     for (int part = 0; part < kSymParts; ++part) c.occ_sym_multi[part] = occupancy_sym_multi<double>(part);
     c.occ_sym_max = occupancy_sym_max<double>();
     if (const char* env = std::getenv("SPG_TILE_PREFIX_MIN")) c.tile_prefix_min = std::max(1, std::atoi(env));
+    if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::max(0, std::atoi(env));
     for (int v = 0; v < kNumLdsVariants; ++v) {
         c.occ_num[0][v] = occupancy_symnum_bin<float>(v);
         c.occ_num[1][v] = occupancy_symnum_bin<double>(v);
@@ -1149,6 +1153,7 @@ struct Job : JobBase {
             p.bref = bref + entry_base;
             p.m = A[i].m;
             p.n = B[i].n;
+            p.wide = B[i].nnz >= c.wide_min ? 1 : 0;
             if (batch) {
                 const int first = static_cast<int>(tiles.size());
                 for (int r0 = 0; r0 < A[i].m; r0 += kTileRows)

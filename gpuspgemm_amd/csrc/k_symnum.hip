@@ -10,7 +10,8 @@
 //      num.cuh:28-41) and add the product there (num.cuh:104-116);
 //   4. write the values to C.val.
 // Fusing the two passes keeps the sorted column list in LDS between them,
-// so C.col is written once and never read back.  A row whose products fit
+// so C.col is written once and never read back.  Rows of 64 lanes add their
+// values in the hash table itself (symnum_wave_row).  A row whose products fit
 // in one chunk and in the lanes' PMAX register slots keeps (column, a*b)
 // in registers from step 1 to step 3 and reads A and B only once.
 #include "spg_kernels.hpp"
@@ -170,6 +171,104 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     gsync<L>();  // LDS is reused by the next unit
 }
 
+// A row of one wave (64 lanes).  The hash table carries a value beside every
+// key: a product is looked up (or its column inserted) once and its value
+// added to its slot right away, so the row's products are walked once, however
+// many there are, and nothing of them outlives the walk.  (The narrower
+// variants keep or re-read the products and binary-search the sorted list for
+// each: seven dependent LDS reads a product at P = 128.)  The occupied slots
+// are then compacted, sorted in registers, and every sorted column picks its
+// value up from the table, one probe per entry of C instead of one search per
+// product.  Bound by VALU issue and LDS latency: four slots a round and 64
+// VGPRs (eight waves per SIMD) beat six or eight slots at six or five waves
+// by 7 and 18 %, and a table of 4P slots (fewer probes, five waves) by 6 %.
+// 96^3 stencil (729 products and 125 entries a row, FP64): 2.70 ms for the
+// launch with staged products and binary searches, 1.23 ms so.
+template <typename V, int P, int T, int N>
+__device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowItem* __restrict__ items, int idx,
+                                                WaveRow<V, P, T>& row, DevMeta* meta) {
+    constexpr int E = P / kWave;
+    constexpr int S = T / kWave;
+    const int lane = lane_id();
+    {
+        typedef int Words __attribute__((vector_size(16)));
+        Words* k = reinterpret_cast<Words*>(row.keys);
+        Words* v = reinterpret_cast<Words*>(row.vals);
+#pragma unroll
+        for (int i = 0; i < T / (4 * kWave); ++i) k[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+#pragma unroll
+        for (int i = 0; i < T * static_cast<int>(sizeof(V)) / (16 * kWave); ++i)
+            v[i * kWave + lane] = Words{0, 0, 0, 0};
+    }
+    const RowItem it = load_item(items, idx);
+    const GProb<V> Pr = ps.get(uniform(it.inst));
+    const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+    wave_sync();
+    wave_products<V, N, true>(W, uniform(it.a0), uniform(it.a1), &row.walk,
+                              [&](const int(&key)[N], const V(&prod)[N], const bool(&ok)[N]) {
+                                  uint32_t h[N];
+                                  table_slots<T>(row.keys, key, ok, h);
+#pragma unroll
+                                  for (int j = 0; j < N; ++j)
+                                      if (ok[j]) lds_add(row.vals + h[j], prod[j]);
+                              });
+    wave_sync();
+
+    // the occupied slots, S consecutive ones to a lane, in front of each other
+    int key[S];
+    int mine = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        key[s] = row.keys[lane * S + s];
+        mine += key[s] != kEmpty ? 1 : 0;
+    }
+    const int incl = wave_incl_scan(mine);
+    const int found = wave_last(incl);
+    int pos = incl - mine;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (key[s] != kEmpty) {
+            if (pos < P) row.cols[pos] = key[s];
+            ++pos;
+        }
+    wave_sync();
+    const int cn = uniform(it.cn);
+    if (lane == 0 && cn != found) atomicOr(&meta->flags.v, kFlagMismatch);
+    const int w = min(min(found, P), cn);
+    int x[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) {
+        x[s] = row.cols[lane * E + s];
+        if (lane * E + s >= found) x[s] = INT_MAX;
+    }
+    wave_sort<E>(x);
+    const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);
+    const auto cval = uniform_ptr(Pr.c_val) + uniform(it.c0);
+#pragma unroll
+    for (int s = 0; s < E; ++s)
+        if (lane * E + s < w) {
+            ccol[lane * E + s] = x[s];
+            cval[lane * E + s] = row.vals[table_find<T>(row.keys, x[s])];
+        }
+    wave_sync();  // LDS is reused by the next row
+}
+
+// The rows [first, end) of one unit of variant VV.
+template <typename V, int VV>
+__device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem* __restrict__ items, int first,
+                                            int end, int* smem, int* s_tmp, DevMeta* meta) {
+    constexpr NumVariant kV = kNumVariants[VV];
+    if constexpr (num_wave_row(kV)) {
+        const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+        if (first + wave < end)
+            symnum_wave_row<V, kV.p, kV.t, kV.pmax>(ps, items, first + wave,
+                                                    reinterpret_cast<WaveRow<V, kV.p, kV.t>*>(smem)[wave], meta);
+    } else {
+        symnum_rows<V, kV.wg, kV.r, kV.p, kV.ec, kV.pmax>(ps, items, first, end, smem, s_tmp, meta);
+    }
+}
+
 // One launch per fused variant over the units (R rows each) of one bin; the
 // host launches a workgroup per unit (residency is the hardware's), and the
 // unit of a workgroup is chosen so that consecutive units stay on one XCD.
@@ -183,8 +282,7 @@ __global__ __launch_bounds__(kNumVariants[VV].wg) SPG_WAVES_PER_EU(kNumMinWaves[
     const int units = (count + kV.r - 1) / kV.r;
     const UnitRange ur = xcd_units(units);
     for (int u = ur.first; u < ur.end; u += ur.stride)
-        symnum_rows<V, kV.wg, kV.r, kV.p, kV.ec, kV.pmax>(ps, items, item_off + u * kV.r, item_off + count, smem,
-                                                          s_tmp, meta);
+        symnum_unit<V, VV>(ps, items, item_off + u * kV.r, item_off + count, smem, s_tmp, meta);
 }
 
 #define SPG_NUM_VARIANTS(X) \
@@ -213,9 +311,7 @@ __global__ __launch_bounds__(256) SPG_WAVES_PER_EU(kNumMultiMinWaves[SET]) void 
         if constexpr (num_multi_set(v) == SET) {                                                            \
             static_assert(kNumVariants[v].wg == 256, "merged launches run 256-thread variants");           \
             if (mb.off[b] + k * kNumVariants[v].r < end)                                                    \
-                symnum_rows<V, 256, kNumVariants[v].r, kNumVariants[v].p, kNumVariants[v].ec,               \
-                            kNumVariants[v].pmax>(ps, items, mb.off[b] + k * kNumVariants[v].r, end, smem, s_tmp, \
-                                                  meta);                                                    \
+                symnum_unit<V, v>(ps, items, mb.off[b] + k * kNumVariants[v].r, end, smem, s_tmp, meta);    \
         }                                                                                                   \
         break;
     switch (mb.variant[b]) {

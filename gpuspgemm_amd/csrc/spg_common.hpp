@@ -55,6 +55,7 @@ struct Prob {
     long long* bref;
     int32_t m;
     int32_t n;
+    int32_t wide;  // B's columns or values may reach past 4 GiB: byte offsets need 64 bits
 };
 
 // An entry's row of B packed in one word: start in the low half, length in
@@ -100,6 +101,7 @@ struct GProb {
     long long SPG_GLOBAL* bref;
     int32_t m;
     int32_t n;
+    int32_t wide;
 };
 
 // (R: a Prob lvalue in any address space)
@@ -108,7 +110,7 @@ __device__ __forceinline__ GProb<V> global_view(R&& p) {
     return GProb<V>{to_global(p.a_rpt), to_global(p.a_col), to_global(p.a_val), to_global(p.b_rpt),
                     to_global(p.b_col), to_global(p.b_val), to_global(p.c_rpt), to_global(p.c_col),
                     to_global(p.c_val), to_global(p.nip),   to_global(p.bref),  p.m,
-                    p.n};
+                    p.n,                p.wide};
 }
 
 // Tile of a row-parallel pass: instance, first row, row count, index of the

@@ -9,6 +9,7 @@
 #pragma once
 
 #include "spg_common.hpp"
+#include "spg_wave.hpp"
 
 namespace spg {
 
@@ -17,7 +18,11 @@ struct SymVariant {
 };
 struct NumVariant {
     int wg, r, p, ec, pmax;  // ... p = sorted-list capacity (the hash table has 2p slots)
+    int t;                   // table slots of the one-wave rows
 };
+// Rows of one wave each (wg / r == 64): see symnum_wave_row.
+constexpr bool num_wave_row(const NumVariant& v) { return v.wg / v.r == kWave; }
+
 
 // Symbolic (count) variants.  0..8 run inside one multi-bin launch of 256
 // threads; 9 is the largest LDS table with overflow detection
@@ -53,7 +58,7 @@ constexpr int sym_part(int variant) { return variant < kSymPartHi[0] ? 0 : (vari
 // per row; the tuner picks among them per bin.
 constexpr NumVariant kNumVariants[] = {
     {256, 256, 8, 4, 16},   {256, 128, 16, 4, 16}, {256, 64, 32, 8, 16},  {256, 32, 64, 16, 16},
-    {256, 16, 128, 32, 16}, {256, 4, 128, 64, 12}, {256, 4, 512, 64, 16}, {256, 1, 1024, 256, 8},
+    {256, 16, 128, 32, 16}, {256, 4, 128, 64, 4, 256}, {256, 4, 256, 64, 4, 512},  {256, 1, 1024, 256, 8},
     {256, 1, 2048, 256, 8}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
     {256, 16, 32, 16, 4},   {256, 8, 64, 32, 4},   {256, 64, 8, 8, 4},    {256, 128, 8, 4, 8},
     {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},
@@ -66,7 +71,7 @@ constexpr int kNumLdsVariants = 19;  // variants with an LDS kernel (0..18)
 // the variant had with the one-by-one fetch, and the compiler schedules
 // the batch within it.  Measured on gfx950: the 96^3 stencil's fused pass
 // 3.23 -> 2.81 ms, the power-law's 198k-row bin 70 -> 53 us.
-constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 4, 3, 4, 3, 4, 8, 8, 7, 6, 7, 5, 7, 5, 5};
+constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 4, 3, 4, 8, 8, 7, 6, 7, 5, 7, 5, 5};
 constexpr int kNumGlobalVariant = 19;
 
 // Fused variants whose bins share one launch.  Set 0, small rows (256
@@ -118,7 +123,8 @@ constexpr int padded_row_ints(int bytes) {
 // Fused variant (FP64 sizing): table 2p ints (reused for p values), sorted
 // list p ints, chunk metadata when the row has more than one lane.
 constexpr int num_row_ints(const NumVariant& v) {
-    return padded_row_ints(12 * v.p + (v.wg / v.r > 1 ? 16 * v.ec : 0));
+    return num_wave_row(v) ? wave_row_bytes(v.p, v.t, sizeof(double)) / 4
+                           : padded_row_ints(12 * v.p + (v.wg / v.r > 1 ? 16 * v.ec : 0));
 }
 // Symbolic variant: table t ints, chunk metadata without values.
 constexpr int sym_row_ints(const SymVariant& v) {

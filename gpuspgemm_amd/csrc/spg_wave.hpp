@@ -1,0 +1,373 @@
+// Building blocks of the rows that whole waves work on (long rows): a wave
+// walks a row's products 64 to a slot, kSlots slots to a round, and keeps
+// everything that is the same for its 64 lanes (the row, the operands'
+// pointers, product counts) in scalar registers.
+//
+// These passes are bound by the vector instructions they issue per product
+// (a SIMD issues one per 4 cycles), so the helpers below are written by
+// instruction count: prefix sums on DPP operands instead of cross-lane
+// reads through LDS, a 24-bit multiply for the hash (a 32-bit one takes
+// four times as long), 32-bit byte offsets from a scalar base for B's
+// columns and values, and compare-exchanges whose direction is a constant
+// lane mask.
+#pragma once
+
+#include "spg_common.hpp"
+
+namespace spg {
+
+__device__ __forceinline__ int uniform(int v) {
+    return static_cast<int>(__builtin_amdgcn_readfirstlane(static_cast<unsigned>(v)));
+}
+template <typename T>
+__device__ __forceinline__ T SPG_GLOBAL* uniform_ptr(T SPG_GLOBAL* p) {
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned long long lo = static_cast<unsigned>(uniform(static_cast<int>(v)));
+    const unsigned long long hi = static_cast<unsigned>(uniform(static_cast<int>(v >> 32)));
+    return (T SPG_GLOBAL*)(lo | hi << 32);
+}
+
+// The lanes of a constant mask, as a per-lane predicate (no instruction on
+// the vector side).
+__device__ __forceinline__ bool in_mask(unsigned long long mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// Set bits of a wave mask below this lane.
+__device__ __forceinline__ int rank_in(unsigned long long mask) {
+    return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u)));
+}
+
+// Inclusive prefix sum over the wave: four DPP row shifts, then the two row
+// broadcasts.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+    return v;
+}
+// The value of lane 63.
+__device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
+
+// Slot of a column in a table of T <= 2^16 slots: the fraction of
+// column * golden ratio, from the low 24 bits of both factors (columns that
+// differ by a multiple of 2^24 share a slot and probe on).
+template <int T>
+__device__ __forceinline__ uint32_t slot24(int key) {
+    constexpr int kBits = __builtin_ctz(T);
+    static_assert((T & (T - 1)) == 0 && kBits >= 1 && kBits <= 16, "bad table size");
+    constexpr uint32_t kGolden = 0x9E3779u;
+    uint32_t x;
+#if defined(__HIP_DEVICE_COMPILE__)
+    // (from plain code the compiler picks the slower 32-bit multiply)
+    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(x) : "v"(key), "s"(kGolden));
+#else
+    x = (static_cast<uint32_t>(key) & 0xFFFFFFu) * kGolden;
+#endif
+    return (x >> (24 - kBits)) & (T - 1);
+}
+
+// Slots of N keys in an LDS table of T slots (open addressing, linear
+// probing), inserting those that are new.  The probes of all keys advance
+// together, each a compare-and-swap; the lanes still probing are kept as
+// scalar masks, so that a key whose lanes are all done costs nothing more.
+// The table never fills (its row has fewer distinct columns than T).
+template <int T, int N>
+__device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const bool (&ok)[N], uint32_t (&h)[N]) {
+    int old[N];
+    unsigned long long pend[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        h[j] = slot24<T>(key[j]);
+        if (ok[j]) old[j] = atomicCAS(tab + h[j], kEmpty, key[j]);
+    }
+    unsigned long long any = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const bool on = ok[j] && old[j] != kEmpty && old[j] != key[j];
+        h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
+        pend[j] = __ballot(on);
+        any |= pend[j];
+    }
+    while (any) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            if (pend[j] && in_mask(pend[j])) old[j] = atomicCAS(tab + h[j], kEmpty, key[j]);
+        any = 0;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            if (!pend[j]) continue;
+            const bool on = in_mask(pend[j]) && old[j] != kEmpty && old[j] != key[j];
+            h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
+            pend[j] = __ballot(on);
+            any |= pend[j];
+        }
+    }
+}
+
+// Slot of a key that is in the table.
+template <int T>
+__device__ __forceinline__ uint32_t table_find(const int* tab, int key) {
+    uint32_t h = slot24<T>(key);
+    while (lds_load(tab + h) != key) h = (h + 1) & (T - 1);
+    return h;
+}
+
+// Sort of 64 * E keys, lane l holding keys l*E .. l*E + E-1 of the result
+// (ascending): the bitonic network of bitonic_sort_regs for one whole wave,
+// a compare and a select per key and stage.
+template <int LJ>
+__device__ __forceinline__ int wave_xor(int v) {
+    if constexpr (LJ == 1)
+        return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);  // quad_perm [1,0,3,2]
+    else if constexpr (LJ == 2)
+        return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);  // quad_perm [2,3,0,1]
+    else if constexpr (LJ == 8)
+        return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, false);  // row_ror:8
+    else if constexpr (LJ < 32)
+        return __builtin_amdgcn_ds_swizzle(v, (LJ << 10) | 0x1F);
+    else
+        return __shfl_xor(v, LJ);
+}
+
+// Lanes that keep the larger key of their pair at stage (K, J) for key s.
+template <int E, int K, int J>
+constexpr unsigned long long larger_lanes(int s) {
+    unsigned long long m = 0;
+    for (int l = 0; l < kWave; ++l) {
+        const bool asc = ((l * E + s) & K) == 0;
+        const bool lower = (l & (J / E)) == 0;
+        if (lower != asc) m |= 1ull << l;
+    }
+    return m;
+}
+// Lanes whose in-lane pair is ascending at level K.
+template <int E, int K>
+constexpr unsigned long long falling_lanes(int s) {
+    unsigned long long m = 0;
+    for (int l = 0; l < kWave; ++l)
+        if (((l * E + s) & K) != 0) m |= 1ull << l;
+    return m;
+}
+
+template <int E, int K, int J>
+__device__ __forceinline__ void wave_sort_stage(int (&x)[E]) {
+    if constexpr (J >= E) {
+        int other[E];
+#pragma unroll
+        for (int s = 0; s < E; ++s) other[s] = wave_xor<J / E>(x[s]);
+        static_for<0, E>([&](auto si) {
+            constexpr int s = decltype(si)::value;
+            constexpr unsigned long long kLarger = larger_lanes<E, K, J>(s);
+            x[s] = (x[s] < other[s]) != in_mask(kLarger) ? x[s] : other[s];
+        });
+    } else {
+        static_for<0, E>([&](auto si) {
+            constexpr int s = decltype(si)::value;
+            if constexpr ((s & J) == 0) {
+                if constexpr (K < E) {  // the direction is the same for every lane
+                    const int lo = min(x[s], x[s + J]), hi = max(x[s], x[s + J]);
+                    x[s] = (s & K) == 0 ? lo : hi;
+                    x[s + J] = (s & K) == 0 ? hi : lo;
+                } else {
+                    constexpr unsigned long long kFalling = falling_lanes<E, K>(s);
+                    const bool keep = (x[s] < x[s + J]) != in_mask(kFalling);
+                    const int a = x[s], b = x[s + J];
+                    x[s] = keep ? a : b;
+                    x[s + J] = keep ? b : a;
+                }
+            }
+        });
+    }
+}
+template <int E, int K, int J>
+__device__ __forceinline__ void wave_sort_level(int (&x)[E]) {
+    if constexpr (J >= 1) {
+        wave_sort_stage<E, K, J>(x);
+        wave_sort_level<E, K, J / 2>(x);
+    }
+}
+template <int E, int K = 2>
+__device__ __forceinline__ void wave_sort(int (&x)[E]) {
+    if constexpr (K <= kWave * E) {
+        wave_sort_level<E, K, K / 2>(x);
+        wave_sort<E, 2 * K>(x);
+    }
+}
+
+// An entry of A as the wave's lanes read it: a_ik and where its row of B
+// lies (position of the row's first product, minus the entry's product
+// offset in the chunk).
+template <typename V, bool VALS>
+struct WaveEntry;
+template <>
+struct alignas(16) WaveEntry<double, true> {
+    double av;
+    int d, pad;
+};
+template <>
+struct alignas(8) WaveEntry<float, true> {
+    float av;
+    int d;
+};
+template <typename V>
+struct WaveEntry<V, false> {
+    int d;
+};
+
+constexpr int kWaveWords = 32;  // 64-bit words of the entry-start bitmap (a window of 2048 products)
+constexpr int kWavePad = 8;     // zero words after it (a round may end past the window)
+
+// Per-wave LDS of the product walk.
+template <typename V, bool VALS>
+struct alignas(16) WaveChunk {
+    unsigned long long starts[kWaveWords + kWavePad];
+    int before[kWaveWords + kWavePad];  // entries that start before each word (and before the window)
+    WaveEntry<V, VALS> ent[kWave];
+};
+
+// LDS of a fused row of one wave: the hash table of T slots with a value
+// beside every key, and the product walk's metadata, whose place the
+// compacted columns take once the walk is over.
+template <typename V, int P, int T>
+struct alignas(16) WaveRow {
+    V vals[T];
+    int keys[T];
+    union {
+        WaveChunk<V, true> walk;
+        int cols[P];
+    };
+};
+constexpr int wave_row_bytes(int p, int t, int value_size) {
+    const int walk = 8 * (kWaveWords + kWavePad) + 4 * (kWaveWords + kWavePad) + kWave * 2 * value_size;
+    const int cols = 4 * p;
+    return t * (value_size + 4) + (walk > cols ? walk : cols);
+}
+static_assert(sizeof(WaveRow<double, 128, 256>) == wave_row_bytes(128, 256, 8) &&
+                  sizeof(WaveRow<float, 512, 1024>) == wave_row_bytes(512, 1024, 4),
+              "LDS size of a wave's row");
+
+// Where a wave's walk reads (all scalar).
+template <typename V>
+struct WaveOperands {
+    const V SPG_GLOBAL* a_val;
+    const long long SPG_GLOBAL* bref;
+    const int32_t SPG_GLOBAL* b_col;
+    const V SPG_GLOBAL* b_val;
+    bool wide;  // B's arrays may pass 4 GiB: 64-bit offsets
+};
+
+// The products of A's entries [a0, a1), in rounds of N * 64:
+// f(key[N], prod[N], ok[N]).  The wave takes 64 entries at a time, one to a
+// lane; entries with an empty row of B drop out.  A product's entry is the
+// number of entries that start at or before it (less one): the chunk's
+// starts are marked in a bitmap, 64 products to a word and one position
+// early, so that a lane counts the marks below its own bit (two mbcnt on
+// top of the count before the word).  `rounds_first` and
+// `rounds_step` let several waves share a row: this wave takes the rounds
+// rounds_first, rounds_first + rounds_step, ... of every chunk, or, with
+// `by_chunk`, every round of the chunks rounds_first, ... instead.
+template <typename V, int N, bool VALS, bool WIDE, typename F>
+__device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<V, VALS>* wc, F&& f,
+                                                 int first, int step, bool by_chunk) {
+    static_assert(N <= kWavePad, "a round may pass the window by N - 1 words");
+    const int lane = lane_id();
+    const int round0 = by_chunk ? 0 : first, round_step = by_chunk ? 1 : step;
+    for (int ebase = a0 + (by_chunk ? first * kWave : 0); ebase < a1; ebase += by_chunk ? step * kWave : kWave) {
+        const int e = ebase + lane;
+        long long ref = 0;
+        V av = V(0);
+        if (e < a1) {
+            ref = W.bref[e];
+            if constexpr (VALS) av = W.a_val[e];
+        }
+        const int len = bref_len(ref);
+        const int incl = wave_incl_scan(len);
+        const int total = wave_last(incl);
+        const int start = incl - len;
+        const unsigned long long filled = __ballot(len > 0);
+        wave_sync();  // the previous chunk's reads are done
+        if (len > 0) {
+            WaveEntry<V, VALS> w;
+            if constexpr (VALS) w.av = av;
+            w.d = (bref_start(ref) - start) * (WIDE ? 1 : 4);  // narrow: in bytes of b_col, modulo 2^32
+            wc->ent[rank_in(filled)] = w;
+        }
+        for (int win = 0; win < total; win += kWave * kWaveWords) {
+            wave_sync();  // the previous window's reads are done
+            if (lane < kWaveWords + kWavePad) wc->starts[lane] = 0;
+            wave_sync();
+            const int mark = start - 1 - win;
+            const bool marks = len > 0 && start > 0;
+            if (marks && mark >= 0 && mark < kWave * kWaveWords)
+                atomicOr(&wc->starts[mark >> 6], 1ull << (mark & 63));
+            const int earlier = __popcll(__ballot(marks && mark < 0));
+            wave_sync();
+            if (lane < kWave) {
+                const int c = lane < kWaveWords ? __popcll(wc->starts[lane]) : 0;
+                const int up = wave_incl_scan(c);
+                if (lane < kWaveWords + kWavePad) wc->before[lane] = earlier + up - c;
+            }
+            wave_sync();
+            const int in_win = min(total - win, kWave * kWaveWords);
+            const int n_rounds = (in_win + N * kWave - 1) / (N * kWave);
+            for (int r = round0; r < n_rounds; r += round_step) {
+                const int base = r * N * kWave;  // in the window
+                int en[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    const unsigned long long w = wc->starts[r * N + j];
+                    en[j] = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                        static_cast<unsigned>(w >> 32),
+                        __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(w),
+                                                  static_cast<unsigned>(wc->before[r * N + j]))));
+                }
+                bool ok[N];
+                int key[N];
+                V bv[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) {
+                    // a lane past the last product reads B's first entry
+                    const int p0 = base + j * kWave;
+                    ok[j] = lane < in_win - p0;
+                    if constexpr (WIDE) {
+                        const int pos = wc->ent[en[j]].d + lane + (win + p0);
+                        const int at = ok[j] ? pos : 0;
+                        key[j] = W.b_col[at];
+                        if constexpr (VALS) bv[j] = W.b_val[at];
+                    } else {
+                        const uint32_t pos = static_cast<uint32_t>(wc->ent[en[j]].d) + static_cast<uint32_t>(lane * 4) +
+                                             static_cast<uint32_t>((win + p0) * 4);
+                        const uint32_t o = ok[j] ? pos : 0u;
+                        key[j] = *(const int32_t SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_col + o);
+                        if constexpr (VALS)
+                            bv[j] = *(const V SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_val +
+                                                           o * static_cast<uint32_t>(sizeof(V) / 4));
+                    }
+                }
+                V prod[N];
+                if constexpr (VALS) {
+                    V a[N];
+#pragma unroll
+                    for (int j = 0; j < N; ++j) a[j] = wc->ent[en[j]].av;
+#pragma unroll
+                    for (int j = 0; j < N; ++j) prod[j] = a[j] * bv[j];
+                }
+                f(key, prod, ok);
+            }
+        }
+    }
+}
+
+template <typename V, int N, bool VALS, typename F>
+__device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<V, VALS>* wc, F&& f,
+                                              int first = 0, int step = 1, bool by_chunk = true) {
+    if (W.wide)
+        wave_products_at<V, N, VALS, true>(W, a0, a1, wc, f, first, step, by_chunk);
+    else
+        wave_products_at<V, N, VALS, false>(W, a0, a1, wc, f, first, step, by_chunk);
+}
+
+}  // namespace spg

@@ -136,14 +136,34 @@ inline T __shfl_xor(T v, int mask, int width = 64) {
     idx = idx >= ((self + width) & ~(width - 1)) ? self : idx;
     return emu_shfl_any(v, idx);
 }
-// DPP quad permutation (the two patterns the library uses: lane ^ 1 and
-// lane ^ 2 within each quad) and the swizzle bit mode (lane ^ xor within
-// each group of 32: pattern = xor << 10 | and_mask 0x1f).
-inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int, int, bool) {
+// DPP controls the library uses: quad permutations (lane ^ 1 and lane ^ 2
+// within each quad), row_shr:n and row_ror:n within rows of 16 lanes, and
+// the broadcasts of lane 15 of a row to the next row and of lane 31 to the
+// upper half.  Lanes whose row is masked out, or that read no lane, keep
+// `old` (0 with bound_ctrl).
+inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int row_mask, int, bool bound_ctrl) {
     const int self = emu::lane();
-    const int sel = (ctrl >> (2 * (self & 3))) & 3;
-    return emu_shfl_any(v, (self & ~3) | sel);
+    const int row = self >> 4, in_row = self & 15;
+    int src = -1;
+    if (ctrl <= 0xff)
+        src = (self & ~3) | ((ctrl >> (2 * (self & 3))) & 3);
+    else if (ctrl >= 0x111 && ctrl <= 0x11f)
+        src = in_row >= (ctrl & 15) ? self - (ctrl & 15) : -1;
+    else if (ctrl >= 0x121 && ctrl <= 0x12f)
+        src = (row << 4) | ((in_row - (ctrl & 15)) & 15);
+    else if (ctrl == 0x142)
+        src = row > 0 ? (row << 4) - 1 : -1;
+    else if (ctrl == 0x143)
+        src = self >= 32 ? 31 : -1;
+    const int got = emu_shfl_any(v, src < 0 ? self : src);
+    if (!((row_mask >> row) & 1)) return old;
+    return src >= 0 ? got : (bound_ctrl ? 0 : old);
 }
+inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int row_mask, int bank_mask, bool bound_ctrl) {
+    return __builtin_amdgcn_update_dpp(0, v, ctrl, row_mask, bank_mask, bound_ctrl);
+}
+inline int __builtin_amdgcn_readlane(int v, int src) { return emu_shfl_any(v, src); }
+inline bool __builtin_amdgcn_inverse_ballot_w64(unsigned long long mask) { return (mask >> emu::lane()) & 1; }
 inline int __builtin_amdgcn_ds_swizzle(int v, int pattern) {
     const int self = emu::lane();
     const int and_mask = pattern & 0x1f, or_mask = (pattern >> 5) & 0x1f, xor_mask = (pattern >> 10) & 0x1f;

@@ -327,6 +327,21 @@ def _heavy_row_case():
 GLOBAL_TABLES = {0: f"{SYM_MAX} {INT_MAX} {INT_MAX}\n", 1: f"{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
 
 
+@pytest.mark.parametrize("variant", [v for v, (lanes, _, _) in sorted(NUM.items()) if lanes == 64])
+def test_wave_rows_windows_and_wide_offsets(emu, tmp_path, variant):
+    """Fused rows of one wave whose chunks of 64 entries hold more products
+    than one window of the entry-start bitmap (2048), with entries that
+    start before a window and run on into it, A rows of several chunks, and
+    rows filled to the variant's capacity; with B's arrays addressed by 32-
+    and by 64-bit offsets (SPG_WIDE_MIN)."""
+    _, _, p = NUM[variant]
+    table = {1: f"{variant} {INT_MAX} {p}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
+    A = gen.random_csr(7, 150, 0.9, seed=80 + variant)
+    B = gen.random_csr(150, p, 0.5, seed=81 + variant, empty_rows=0.1)
+    run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A, B, tables=table, env={"SPG_WIDE_MIN": "0"}),
+                call(A.astype(np.float32), B.astype(np.float32), "--f32", tables=table, env={"SPG_WIDE_MIN": "0"}))
+
+
 def test_global_paths(emu, tmp_path):
     """The heavy-row case first with the default tables and then with every
     row forced to the global kernels."""
