@@ -83,7 +83,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     constexpr int ROW_INTS = num_row_ints(NumVariant{WG, R, P, EC, PMAX});
     static_assert(WG % R == 0, "bad variant shape");
     static_assert(L <= kWave || R == 1, "a row spans several waves only when it owns the workgroup");
-    static_assert(T * sizeof(int) >= P * sizeof(V), "values must fit in the table's LDS");
+    static_assert(T * sizeof(int) >= P * sizeof(LdsSum), "values must fit in the table's LDS");
     static_assert(ROW_INTS % 2 == 0, "row slots must stay 8-byte aligned");
     using Meta = ChunkMeta<V, EC, true>;
     using KeyMeta = ChunkMeta<V, EC, false>;
@@ -92,7 +92,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     int* tab = smem + slot * ROW_INTS;
     int* cols = tab + T;
     Meta* cm = reinterpret_cast<Meta*>(cols + P);
-    V* vals = reinterpret_cast<V*>(tab);
+    LdsSum* vals = reinterpret_cast<LdsSum*>(tab);
 
     lds_fill<T, L>(tab, kEmpty, lr);
     gsync<L>();
@@ -144,7 +144,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     } else {
         for (int j = lr; j < w; j += L) Pr.c_col[c0 + j] = cols[j];
     }
-    for (int j = lr; j < P; j += L) vals[j] = V(0);
+    for (int j = lr; j < P; j += L) vals[j] = 0;
     gsync<L>();
 
     // binary search of every product's column in the sorted list
@@ -159,7 +159,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
             lower_bound_all<P, G, J0>(cols, k, pos);
 #pragma unroll
             for (int j = 0; j < G; ++j)
-                if (o[J0 + j]) lds_add(vals + pos[j], v[J0 + j]);
+                if (o[J0 + j]) lds_add(vals + pos[j], static_cast<LdsSum>(v[J0 + j]));
         });
     };
     if (fits)
@@ -167,7 +167,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     else
         for_each_round<V, L, EC, PMAX, true>(Pr, a0, a1, lr, cm, s_tmp, accumulate);
     gsync<L>();
-    for (int j = lr; j < w; j += L) Pr.c_val[c0 + j] = vals[j];
+    for (int j = lr; j < w; j += L) Pr.c_val[c0 + j] = static_cast<V>(vals[j]);
     gsync<L>();  // LDS is reused by the next unit
 }
 
@@ -186,7 +186,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
 // launch with staged products and binary searches, 1.23 ms so.
 template <typename V, int P, int T, int N>
 __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowItem* __restrict__ items, int idx,
-                                                WaveRow<V, P, T>& row, DevMeta* meta) {
+                                                WaveRow<P, T>& row, DevMeta* meta) {
     constexpr int E = P / kWave;
     constexpr int S = T / kWave;
     const int lane = lane_id();
@@ -197,7 +197,7 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
 #pragma unroll
         for (int i = 0; i < T / (4 * kWave); ++i) k[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
-        for (int i = 0; i < T * static_cast<int>(sizeof(V)) / (16 * kWave); ++i)
+        for (int i = 0; i < T * static_cast<int>(sizeof(LdsSum)) / (16 * kWave); ++i)
             v[i * kWave + lane] = Words{0, 0, 0, 0};
     }
     const RowItem it = load_item(items, idx);
@@ -206,7 +206,7 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
                             uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
     wave_sync();
     wave_products<V, N, true>(W, uniform(it.a0), uniform(it.a1), &row.walk,
-                              [&](const int(&key)[N], const V(&prod)[N], const bool(&ok)[N]) {
+                              [&](const int(&key)[N], const LdsSum(&prod)[N], const bool(&ok)[N]) {
                                   uint32_t h[N];
                                   table_slots<T>(row.keys, key, ok, h);
 #pragma unroll
@@ -249,7 +249,7 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
     for (int s = 0; s < E; ++s)
         if (lane * E + s < w) {
             ccol[lane * E + s] = x[s];
-            cval[lane * E + s] = row.vals[table_find<T>(row.keys, x[s])];
+            cval[lane * E + s] = static_cast<V>(row.vals[table_find<T>(row.keys, x[s])]);
         }
     wave_sync();  // LDS is reused by the next row
 }
@@ -263,7 +263,7 @@ __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem*
         const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
         if (first + wave < end)
             symnum_wave_row<V, kV.p, kV.t, kV.pmax>(ps, items, first + wave,
-                                                    reinterpret_cast<WaveRow<V, kV.p, kV.t>*>(smem)[wave], meta);
+                                                    reinterpret_cast<WaveRow<kV.p, kV.t>*>(smem)[wave], meta);
     } else {
         symnum_rows<V, kV.wg, kV.r, kV.p, kV.ec, kV.pmax>(ps, items, first, end, smem, s_tmp, meta);
     }

@@ -120,10 +120,10 @@ constexpr int padded_row_ints(int bytes) {
     const int words = (bytes + 7) / 8;
     return 2 * (words % 2 ? words : words + 1);
 }
-// Fused variant (FP64 sizing): table 2p ints (reused for p values), sorted
+// Fused variant: table 2p ints (reused for p sums in double), sorted
 // list p ints, chunk metadata when the row has more than one lane.
 constexpr int num_row_ints(const NumVariant& v) {
-    return num_wave_row(v) ? wave_row_bytes(v.p, v.t, sizeof(double)) / 4
+    return num_wave_row(v) ? wave_row_bytes(v.p, v.t) / 4
                            : padded_row_ints(12 * v.p + (v.wg / v.r > 1 ? 16 * v.ec : 0));
 }
 // Symbolic variant: table t ints, chunk metadata without values.

@@ -200,20 +200,15 @@ __device__ __forceinline__ void wave_sort(int (&x)[E]) {
 // An entry of A as the wave's lanes read it: a_ik and where its row of B
 // lies (position of the row's first product, minus the entry's product
 // offset in the chunk).
-template <typename V, bool VALS>
+template <bool VALS>
 struct WaveEntry;
 template <>
-struct alignas(16) WaveEntry<double, true> {
+struct alignas(16) WaveEntry<true> {
     double av;
     int d, pad;
 };
 template <>
-struct alignas(8) WaveEntry<float, true> {
-    float av;
-    int d;
-};
-template <typename V>
-struct WaveEntry<V, false> {
+struct WaveEntry<false> {
     int d;
 };
 
@@ -221,32 +216,33 @@ constexpr int kWaveWords = 32;  // 64-bit words of the entry-start bitmap (a win
 constexpr int kWavePad = 8;     // zero words after it (a round may end past the window)
 
 // Per-wave LDS of the product walk.
-template <typename V, bool VALS>
+template <bool VALS>
 struct alignas(16) WaveChunk {
     unsigned long long starts[kWaveWords + kWavePad];
     int before[kWaveWords + kWavePad];  // entries that start before each word (and before the window)
-    WaveEntry<V, VALS> ent[kWave];
+    WaveEntry<VALS> ent[kWave];
 };
 
 // LDS of a fused row of one wave: the hash table of T slots with a value
 // beside every key, and the product walk's metadata, whose place the
-// compacted columns take once the walk is over.
-template <typename V, int P, int T>
+// compacted columns take once the walk is over.  Values are summed in double
+// whatever the operands' type (LdsSum).
+template <int P, int T>
 struct alignas(16) WaveRow {
-    V vals[T];
+    LdsSum vals[T];
     int keys[T];
     union {
-        WaveChunk<V, true> walk;
+        WaveChunk<true> walk;
         int cols[P];
     };
 };
-constexpr int wave_row_bytes(int p, int t, int value_size) {
-    const int walk = 8 * (kWaveWords + kWavePad) + 4 * (kWaveWords + kWavePad) + kWave * 2 * value_size;
+constexpr int wave_row_bytes(int p, int t) {
+    const int walk = static_cast<int>(sizeof(WaveChunk<true>));
     const int cols = 4 * p;
-    return t * (value_size + 4) + (walk > cols ? walk : cols);
+    return t * static_cast<int>(sizeof(LdsSum) + sizeof(int)) + (walk > cols ? walk : cols);
 }
-static_assert(sizeof(WaveRow<double, 128, 256>) == wave_row_bytes(128, 256, 8) &&
-                  sizeof(WaveRow<float, 512, 1024>) == wave_row_bytes(512, 1024, 4),
+static_assert(sizeof(WaveRow<128, 256>) == wave_row_bytes(128, 256) &&
+                  sizeof(WaveRow<512, 1024>) == wave_row_bytes(512, 1024),
               "LDS size of a wave's row");
 
 // Where a wave's walk reads (all scalar).
@@ -270,7 +266,7 @@ struct WaveOperands {
 // rounds_first, rounds_first + rounds_step, ... of every chunk, or, with
 // `by_chunk`, every round of the chunks rounds_first, ... instead.
 template <typename V, int N, bool VALS, bool WIDE, typename F>
-__device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<V, VALS>* wc, F&& f,
+__device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                                  int first, int step, bool by_chunk) {
     static_assert(N <= kWavePad, "a round may pass the window by N - 1 words");
     const int lane = lane_id();
@@ -290,7 +286,7 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
         const unsigned long long filled = __ballot(len > 0);
         wave_sync();  // the previous chunk's reads are done
         if (len > 0) {
-            WaveEntry<V, VALS> w;
+            WaveEntry<VALS> w;
             if constexpr (VALS) w.av = av;
             w.d = (bref_start(ref) - start) * (WIDE ? 1 : 4);  // narrow: in bytes of b_col, modulo 2^32
             wc->ent[rank_in(filled)] = w;
@@ -347,13 +343,13 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
                                                            o * static_cast<uint32_t>(sizeof(V) / 4));
                     }
                 }
-                V prod[N];
+                LdsSum prod[N];
                 if constexpr (VALS) {
-                    V a[N];
+                    LdsSum a[N];
 #pragma unroll
                     for (int j = 0; j < N; ++j) a[j] = wc->ent[en[j]].av;
 #pragma unroll
-                    for (int j = 0; j < N; ++j) prod[j] = a[j] * bv[j];
+                    for (int j = 0; j < N; ++j) prod[j] = a[j] * static_cast<LdsSum>(bv[j]);
                 }
                 f(key, prod, ok);
             }
@@ -362,7 +358,7 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
 }
 
 template <typename V, int N, bool VALS, typename F>
-__device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<V, VALS>* wc, F&& f,
+__device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                               int first = 0, int step = 1, bool by_chunk = true) {
     if (W.wide)
         wave_products_at<V, N, VALS, true>(W, a0, a1, wc, f, first, step, by_chunk);
