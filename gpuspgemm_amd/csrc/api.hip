@@ -8,8 +8,7 @@
 // from a device block cache, and a multiply is
 //
 //   nip (with the symbolic binning)
-//   -> sym_multi_small on the main stream || sym_max, sym_multi on two aux
-//      streams (forked and joined with events)
+//   -> sym_multi, sym_max (exact counts)
 //   -> scan_count, scan_apply
 //   -> one kernel copies the counters to pinned host memory, zeroes them
 //      and signals; the host polls the signal (one synchronisation)
@@ -55,12 +54,6 @@ namespace {
 // with hipGetSymbolAddress, and uses only that address.
 constexpr size_t kNoAllocScratch = size_t(256) << 20;
 static __device__ __align__(256) char scratch[kNoAllocScratch];
-
-// Products whose mean NIP per row, estimated from the operands' densities,
-// is at most this many queue the symbolic pass's small-table part first
-// (power-law 10^6 rows: 8.6, measured 0.325 -> 0.305 ms; the 96^3 stencil,
-// 704, keeps the other order: 3.9 ms against 4.4 with this one).
-constexpr double kSmallFirstNip = 32;
 
 // Tile count (of 2048 rows) from which the scan stage scans the tile sums
 // once (k_tile_prefix, one workgroup: ~2 us per 1024 tiles) instead of
@@ -348,7 +341,7 @@ struct alignas(64) DoneWord {
 };
 
 // The device resources of one multiply in flight: aux streams that the
-// symbolic phase forks onto and the fused-pass launches are spread over,
+// fused-pass launches are spread over,
 // events for the forks and joins, a scratch arena that only grows, and
 // pinned host memory for the read-backs.  The main stream is the caller's
 // (a thread's default stream for the synchronous calls) or the lane's own.
@@ -466,7 +459,7 @@ struct Context {
     std::mutex mu;  // tables, the lane map, profiling records
     BinTable sym{};
     BinTable num{};
-    int occ_sym_multi[kSymParts] = {1, 1, 1}, occ_sym_max = 1;
+    int occ_sym_multi = 1, occ_sym_max = 1;
     int occ_num[2][kNumLdsVariants] = {};
     // tiles from which the scan reads each tile's prefix off one scanned
     // array instead of summing the earlier tiles per workgroup (quadratic
@@ -530,14 +523,15 @@ void default_tables(BinTable& sym, BinTable& num) {
 
 // A symbolic table is a run of multi-bin variants followed by the max
 // variant with caps INT_MAX.  Each multi bin's NIP cap must stay below its
-// table size, so a row's distinct columns (<= NIP) never fill the table.
+// table size, so a row's distinct columns (<= NIP) never fill the table
+// (variant 8 detects that itself).
 spg_status check_sym_table(const BinTable& t) {
     if (t.n < 1 || t.n > kMaxBins) return fail(SPG_ERR_INVALID_ARGUMENT, "symbolic table: bad bin count");
     for (int b = 0; b + 1 < t.n; ++b) {
         const int v = t.variant[b];
         if (v < 0 || v >= kSymMultiVariants)
             return fail(SPG_ERR_INVALID_ARGUMENT, "symbolic table: bins before the last must use the multi-bin variants");
-        if (t.nip_cap[b] >= kSymVariants[v].t || t.nip_cap[b] < 1)
+        if ((t.nip_cap[b] >= kSymVariants[v].t && v != kSymOverVariant) || t.nip_cap[b] < 1)
             return fail(SPG_ERR_INVALID_ARGUMENT, "symbolic table: NIP cap must be below the variant's table size");
     }
     if (t.variant[t.n - 1] != kSymMaxVariant || t.nip_cap[t.n - 1] != INT_MAX)
@@ -594,7 +588,7 @@ spg_status ensure_context(Context*& out) {
     c.clock_khz = prop.clockRate;
     c.global_mem = prop.totalGlobalMem;
     if (c.lds < kNumBigLds + 1024 ||
-        c.lds < kSymVariants[kSymMaxVariant].t * 4 + 8 * kSymVariants[kSymMaxVariant].ec + 1024)
+        c.lds < 4 * sym_row_ints(kSymVariants[kSymMaxVariant]) + 1024)
         return fail(SPG_ERR_UNSUPPORTED_DEVICE, "device offers less LDS per workgroup than the kernels need");
     SPG_TRY(lane_create(c.lane));
     SPG_TRY(lane_create(c.noalloc_lane));
@@ -603,7 +597,7 @@ spg_status ensure_context(Context*& out) {
     default_tables(c.sym, c.num);
     SPG_TRY(check_sym_table(c.sym));  // a stale tuned_tables.inc fails here, loudly
     SPG_TRY(check_num_table(c.num));
-    for (int part = 0; part < kSymParts; ++part) c.occ_sym_multi[part] = occupancy_sym_multi<double>(part);
+    c.occ_sym_multi = std::min(occupancy_sym_multi<double>(), occupancy_sym_multi<float>());
     c.occ_sym_max = occupancy_sym_max<double>();
     if (const char* env = std::getenv("SPG_TILE_PREFIX_MIN")) c.tile_prefix_min = std::max(1, std::atoi(env));
     if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::max(0, std::atoi(env));
@@ -815,7 +809,6 @@ struct Job : JobBase {
     std::vector<Tile> tiles;
     ProbSet<V> ps{};
     long long total_rows = 0;
-    bool small_first = false;  // the symbolic launches in the order of short products (front())
     int n_tiles = 0;
     bool batch = false;
     bool empty = false;
@@ -916,56 +909,16 @@ struct Job : JobBase {
         prof.begin("nip", total_rows, n_tiles, s);
         launch_nip<V>(ps, sym, meta, items1, static_cast<int>(total_rows), s);
         prof.end();
-        // The launches count disjoint rows, on three streams: the part of the
-        // two largest multi-bin tables (rows of a workgroup each, few of
-        // them) on the first aux stream; with the small-table part in use,
-        // the mid-table part on the second aux stream (its workgroups take
-        // the CUs that the small-table grid leaves as its last units drain);
-        // the remaining part on the main stream.  The largest-table bin
-        // (139 KB of LDS a workgroup) goes where its workgroups find free
-        // CUs.  Rows of short products (small_first: a mean NIP per row of
-        // at most kSmallFirstNip, estimated from the operands' densities)
-        // fill the small-table part, the longest launch: it is queued first,
-        // right behind k_nip on the main stream, and the largest-table bin
-        // after it there.  Otherwise the largest-table bin is queued first,
-        // on the first aux stream, while the CUs are still free (its
-        // workgroups without a row exit at once; queued behind the
-        // multi-bin grids they were measured to hold back the mid-table
-        // launch of the stencil by a third), and its part follows it.
         const int n_multi = sym.n - 1;
-        bool part_used[kSymParts] = {};
-        for (int b = 0; b < n_multi; ++b) part_used[sym_part(sym.variant[b])] = true;
-        const bool split = part_used[0] && part_used[1];
-        static const char* const kPartName[kSymParts] = {"sym_multi_small", "sym_multi", "sym_multi_large"};
-        auto part_stream = [&](int part) { return part == 2 ? L.aux[0] : (split && part == 1 ? L.aux[1] : s); };
-        auto queue_part = [&](int part) {
-            const hipStream_t where = part_stream(part);
-            int grid = c.cus * c.occ_sym_multi[part];
-            grid = (grid + kXcds - 1) / kXcds * kXcds;
-            prof.begin(kPartName[part], total_rows, grid, where);
-            launch_sym_multi<V>(part, ps, items1, static_cast<int>(total_rows), sym, n_multi, meta, grid, where);
-            prof.end();
-        };
-        auto queue_max = [&](hipStream_t where) {
-            const int grid = c.cus * c.occ_sym_max;
-            prof.begin("sym_max", 0, grid, where);
-            launch_sym_max<V>(ps, items1, static_cast<int>(total_rows), sym, sym.n - 1, meta, fail_items, fail_off,
-                              grid, where);
-            prof.end();
-        };
-        SPG_HIP(hipEventRecord(L.ev_ready, s));
-        int main_part = -1;  // the part queued on the main stream
-        for (int part : {0, 1})
-            if (main_part < 0 && part_used[part] && part_stream(part) == s) main_part = part;
-        if (small_first && main_part >= 0) queue_part(main_part);
-        SPG_HIP(hipStreamWaitEvent(L.aux[0], L.ev_ready, 0));
-        if (!small_first) queue_max(L.aux[0]);
-        if (split) SPG_HIP(hipStreamWaitEvent(L.aux[1], L.ev_ready, 0));
-        for (int part : {2, 1, 0})
-            if (part_used[part] && !(small_first && part == main_part)) queue_part(part);
-        if (small_first) queue_max(s);
-        SPG_HIP(join(L.aux[0], L.ev_done[0], s));
-        if (split) SPG_HIP(join(L.aux[1], L.ev_done[1], s));
+        int grid = c.cus * c.occ_sym_multi;
+        grid = (grid + kXcds - 1) / kXcds * kXcds;
+        prof.begin("sym_multi", total_rows, grid, s);
+        launch_sym_multi<V>(ps, items1, static_cast<int>(total_rows), sym, n_multi, meta, grid, s);
+        prof.end();
+        grid = c.cus * c.occ_sym_max;
+        prof.begin("sym_max", 0, grid, s);
+        launch_sym_max<V>(ps, items1, static_cast<int>(total_rows), n_multi, meta, fail_items, fail_off, grid, s);
+        prof.end();
         return SPG_OK;
     }
 
@@ -993,7 +946,7 @@ struct Job : JobBase {
     // contents (operand descriptors, tiles) are copied from pinned host
     // memory by the phase itself and so are not part of it.
     std::vector<int64_t> signature(int phase) const {
-        std::vector<int64_t> k{phase, static_cast<int64_t>(sizeof(V)), count, n_tiles, total_rows, small_first,
+        std::vector<int64_t> k{phase, static_cast<int64_t>(sizeof(V)), count, n_tiles, total_rows,
                                reinterpret_cast<int64_t>(L.scratch), reinterpret_cast<int64_t>(L.h_stage)};
         const BinTable& t = phase == 0 ? sym : num;
         k.push_back(t.n);
@@ -1070,12 +1023,6 @@ struct Job : JobBase {
             }
         }
         nnz.assign(count, 0);
-        {
-            double est_nip = 0;  // NIP of all rows if B's entries were spread evenly over its rows
-            for (int i = 0; i < count; ++i)
-                if (B[i].m > 0) est_nip += static_cast<double>(A[i].nnz) * B[i].nnz / B[i].m;
-            small_first = est_nip <= kSmallFirstNip * static_cast<double>(total_rows);
-        }
         // graph replay reads the descriptors from device memory in every call
         batch = count > 1 || graphs;
         if (total_rows >= INT_MAX) return failed(fail(SPG_ERR_OVERFLOW, "total row count exceeds int32"));

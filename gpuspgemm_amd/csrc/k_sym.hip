@@ -1,10 +1,11 @@
 // Symbolic count: exact nnz of every row of C from an open-addressing hash
 // table of the row's B columns (sym1.cuh:28-306), written into c_rpt.
 //
-// A workgroup unit holds R rows; each row owns L = WG/R consecutive lanes
-// that enumerate its products flat (spg_rows.hpp) and insert their columns
-// into the row's LDS table.  Rows that overflow the largest table are
-// recounted in global memory.
+// A workgroup unit holds R rows; a row owns L = WG/R consecutive lanes of a
+// wave (spg_rows.hpp), a wave or the workgroup (spg_wave.hpp), which walk its
+// products and insert their columns into the row's LDS table.  Rows that
+// overflow a table move on to the next larger one, in the end to global
+// memory.
 #include "spg_kernels.hpp"
 #include "spg_rows.hpp"
 
@@ -50,58 +51,164 @@ __device__ __forceinline__ void sym_rows(const ProbSet<V>& ps, const int2* __res
     gsync<L>();  // the table is reused by the next unit
 }
 
-#define SPG_SYM_CASE(v)                                                                                   \
-    case v:                                                                                               \
-        if constexpr (v >= LO && v < HI)                                                                  \
-            sym_rows<V, kMultiThreads, kSymVariants[v].r, kSymVariants[v].t, kSymVariants[v].ec,          \
-                     kSymVariants[v].pmax>(ps, bin_items, first, end, smem, s_tmp);                       \
-        break;
-
-// LDS of a multi-bin launch over variants [LO, HI).
-template <int LO, int HI>
-constexpr int sym_multi_lds() {
-    int m = 0;
-    for (int i = LO; i < HI; ++i) {
-        const int b = 4 * kSymVariants[i].r * sym_row_ints(kSymVariants[i]);
-        m = m > b ? m : b;
+// Rows of one wave each (tables of T slots): rows idx, idx + step, ... below
+// end of the bin's list.  A wave walks a row's products (wave_products) and
+// counts its inserts in a scalar register.  A row starts with a chain of
+// dependent loads (its item, its bounds in A, its entries, B's columns), so
+// the next row's item and bounds are fetched while this one is counted.
+template <typename V, int T, int N>
+__device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* __restrict__ items, int idx, int step,
+                                              int end, int* smem) {
+    typedef int Words __attribute__((vector_size(16)));
+    const int lane = lane_id();
+    int* tab = smem;
+    auto* walk = reinterpret_cast<WaveChunk<false>*>(smem + T);
+    if (idx >= end) return;
+    int2 it = items[idx];
+    int inst = uniform(it.x), row = uniform(it.y);
+    GProb<V> P = ps.get(inst);
+    int a0 = uniform(P.a_rpt[row]), a1 = uniform(P.a_rpt[row + 1]);
+    while (true) {
+        const bool more = idx + step < end;
+        const int2 it_next = items[more ? idx + step : idx];
+#pragma unroll
+        for (int i = 0; i < T / (4 * kWave); ++i)
+            reinterpret_cast<Words*>(tab)[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+        const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide) != 0};
+        wave_sync();
+        const int inst_next = uniform(it_next.x), row_next = uniform(it_next.y);
+        const GProb<V> P_next = ps.get(inst_next);
+        const int b0 = P_next.a_rpt[row_next], b1 = P_next.a_rpt[row_next + 1];
+        int n = 0;
+        wave_products<V, N, false>(W, a0, a1, walk, [&](const int(&key)[N], const LdsSum(&)[N], const bool(&ok)[N]) {
+            uint32_t h[N];
+            table_slots<T, N, true>(tab, key, ok, h, n);
+        });
+        if (lane == 0) P.c_rpt[row] = n;
+        if (!more) break;
+        wave_sync();  // the table is reused by the next row
+        idx += step;
+        inst = inst_next;
+        row = row_next;
+        P = P_next;
+        a0 = uniform(b0);
+        a1 = uniform(b1);
     }
-    return m;
 }
 
-// One launch serves the bins among [0, n_multi) of the symbolic table whose
-// variant lies in [LO, HI).  Bin sizes are read on the device, so the
-// launch needs no host round trip; the grid is persistent and walks the
-// units of its bins.  The small-table variants get a launch of their own:
-// a kernel takes the register budget of its largest variant, and theirs is
-// far smaller, so twice as many of their waves fit on a CU.
-template <typename V, int LO, int HI>
-__global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves[sym_part(LO)]) void k_sym_multi(ProbSet<V> ps, const int2* __restrict__ items,
-                                                             int bin_cap, BinTable sym, int n_multi,
-                                                             const DevMeta* __restrict__ meta) {
-    static_assert(sym_multi_lds<LO, HI>() <= kSymMultiLds, "symbolic multi-bin LDS budget");
-    __shared__ __align__(16) int smem[sym_multi_lds<LO, HI>() / 4];
-    __shared__ int s_tmp[kMultiThreads / kWave];
-    __shared__ int s_unit[kMaxBins + 1];
-    __shared__ int s_cnt[kMaxBins];
-    if (threadIdx.x == 0) {
-        int units = 0;
-        for (int b = 0; b < n_multi; ++b) {
-            const int c = meta->sym_count[b].v;
-            const bool mine = sym.variant[b] >= LO && sym.variant[b] < HI;
-            s_cnt[b] = c;
-            s_unit[b] = units;
-            if (mine) units += (c + sym.rows[b] - 1) / sym.rows[b];
-        }
-        s_unit[n_multi] = units;
-    }
+// A row of a whole workgroup: every wave walks a share of the products on
+// its own (no barrier inside the walk), all insert into one table.  LIMIT >
+// 0: a wave stops inserting once the row has more than LIMIT distinct
+// columns; returns the count (above LIMIT: too many), the same on every lane.
+template <typename V, int WG, int T, int N, int LIMIT>
+__device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* smem) {
+    typedef int Words __attribute__((vector_size(16)));
+    constexpr int kWaves = WG / kWave;
+    const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+    int* tab = smem;
+    auto* walk = reinterpret_cast<WaveChunk<false>*>(smem + T);
+    int* total = reinterpret_cast<int*>(walk + kWaves);
+#pragma unroll
+    for (int i = 0; i < T / (4 * WG); ++i)
+        reinterpret_cast<Words*>(tab)[i * WG + threadIdx.x] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+    if (threadIdx.x == 0) *total = 0;
+    const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide) != 0};
+    const int a0 = uniform(P.a_rpt[row]), a1 = uniform(P.a_rpt[row + 1]);
+    const int nip = uniform(P.nip[row]);
     __syncthreads();
-    const UnitRange ur = xcd_units(s_unit[n_multi]);
-    for (int u = ur.first; u < ur.end; u += ur.stride) {
-        int b = 0;
-        while (u >= s_unit[b + 1]) ++b;
+    int added = 0;
+    auto report = [&]() {
+        if (lane_id() == 0 && added) atomicAdd(total, added);
+        added = 0;
+    };
+    wave_products<V, N, false>(
+        W, a0, a1, walk + wave,
+        [&](const int(&key)[N], const LdsSum(&)[N], const bool(&ok)[N]) -> bool {
+            if constexpr (LIMIT > 0) {
+                if (uniform(lds_load(total)) > LIMIT) return false;
+            }
+            uint32_t h[N];
+            table_slots<T, N, true>(tab, key, ok, h, added);
+            if constexpr (LIMIT > 0) report();
+            return true;
+        },
+        wave, kWaves, wave_by_chunk<kWaves>(a1 - a0, nip));
+    report();
+    __syncthreads();
+    const int n = *total;
+    __syncthreads();  // the table and the total are reused by the next row
+    return n;
+}
+
+template <int VV>
+constexpr int sym_unit_lds() {
+    return 4 * kSymVariants[VV].r * sym_row_ints(kSymVariants[VV]);
+}
+
+// The units k0, k0 + step, ... below k_end (kV.r rows each) of a bin of
+// variant VV.
+template <typename V, int VV>
+__device__ __forceinline__ void sym_units(const ProbSet<V>& ps, const int2* __restrict__ bin_items, int k0, int step,
+                                          int k_end, int count, int* smem, int* s_tmp, int2* over_items,
+                                          DevMeta* meta) {
+    constexpr SymVariant kV = kSymVariants[VV];
+    const int end = min(count, k_end * kV.r);
+    if constexpr (sym_is_wave(kV)) {
+        const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+        sym_wave_rows<V, kV.t, kV.pmax>(ps, bin_items, k0 * kV.r + wave, step * kV.r, end,
+                                        smem + wave * sym_row_ints(kV));
+    } else if constexpr (sym_is_group(kV)) {
+        constexpr int kLimit = VV == kSymOverVariant ? kSymOverThreshold : 0;
+        for (int k = k0; k < end; k += step) {
+            const int2 it = bin_items[k];
+            const GProb<V> P = ps.get(uniform(it.x));
+            const int row = uniform(it.y);
+            const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kLimit>(P, row, smem);
+            if (threadIdx.x == 0) {
+                if (kLimit > 0 && n > kLimit)
+                    over_items[atomicAdd(&meta->over_count.v, 1)] = it;
+                else
+                    P.c_rpt[row] = n;
+            }
+        }
+    } else {
+        for (int first = k0 * kV.r; first < end; first += step * kV.r)
+            sym_rows<V, kV.wg, kV.r, kV.t, kV.ec, kV.pmax>(ps, bin_items, first, end, smem, s_tmp);
+    }
+}
+
+// One launch serves the bins [0, n_multi) of the symbolic table.  Bin sizes
+// are read on the device, so the launch needs no host round trip; the grid
+// is persistent.  Every XCD takes a contiguous slice of every bin, the bins
+// of long rows first, and its workgroups deal the slices' units among
+// themselves.  One kernel for all variants (72 VGPRs and 23 KB of LDS, seven
+// waves per SIMD) keeps the whole symbolic phase on one stream: in three
+// launches on three streams, the fork cost 7 to 14 us and the join 10 to 58.
+template <typename V>
+__global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves) void k_sym_multi(
+    ProbSet<V> ps, int2* __restrict__ items, int bin_cap, BinTable sym, int n_multi, DevMeta* __restrict__ meta) {
+    __shared__ __align__(16) int smem[max_sym_multi_lds() / 4];
+    __shared__ int s_tmp[kMultiThreads / kWave];
+    __shared__ int s_cnt[kMaxBins];
+    if (static_cast<int>(threadIdx.x) < n_multi) s_cnt[threadIdx.x] = meta->sym_count[threadIdx.x].v;
+    __syncthreads();
+    const int xcd = blockIdx.x % kXcds;
+    const int step = gridDim.x / kXcds;
+    int2* over_items = items + static_cast<long long>(sym.n - 1) * bin_cap + meta->sym_count[sym.n - 1].v;
+    int k0 = blockIdx.x / kXcds;  // this workgroup's first unit in the XCD's slice of the bin
+    for (int b = n_multi - 1; b >= 0; --b) {
+        const int count = s_cnt[b];
+        const int per = ((count + sym.rows[b] - 1) / sym.rows[b] + kXcds - 1) / kXcds;  // units of the slice
+        if (k0 >= per) {
+            k0 -= per;
+            continue;
+        }
         const int2* bin_items = items + static_cast<long long>(b) * bin_cap;  // bin b's list
-        const int first = (u - s_unit[b]) * sym.rows[b];
-        const int end = s_cnt[b];
+        const int first = xcd * per;
+#define SPG_SYM_CASE(v)                                                                                            \
+    case v:                                                                                                        \
+        sym_units<V, v>(ps, bin_items, first + k0, step, first + per, count, smem, s_tmp, over_items, meta);       \
+        break;
         switch (sym.variant[b]) {
             SPG_SYM_CASE(0)
             SPG_SYM_CASE(1)
@@ -115,17 +222,13 @@ __global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves[s
             default:
                 break;
         }
-        // Consecutive units may belong to bins with different LDS layouts,
-        // and rows of L <= 64 lanes only synchronise inside their wave: no
-        // wave may start a unit of another layout while another wave still
-        // uses this one.  Units of the same variant give every wave the same
-        // LDS slots, so between them the waves run on without a barrier.
-        const int un = u + ur.stride;
-        if (un < ur.end) {
-            int bn = b;
-            while (un >= s_unit[bn + 1]) ++bn;
-            if (sym.variant[bn] != sym.variant[b]) __syncthreads();
-        }
+#undef SPG_SYM_CASE
+        k0 += (per - k0 + step - 1) / step * step - per;
+        // The next bin may lay out LDS differently, and rows of L <= 64 lanes
+        // only synchronise inside their wave: no wave may start on it while
+        // another wave still uses this one.  Units of one bin give every
+        // wave the same LDS slots, so between them the waves run on.
+        __syncthreads();
     }
 }
 
@@ -138,56 +241,24 @@ __global__ __launch_bounds__(1024) void k_sym_max(ProbSet<V> ps, const int2* __r
                                                   int bin, DevMeta* __restrict__ meta,
                                                   int2* __restrict__ fail_items, long long* __restrict__ fail_off) {
     constexpr SymVariant kV = kSymVariants[kSymMaxVariant];
-    constexpr int T = kV.t;
-    constexpr int WG = 1024;
-    constexpr int EC = kV.ec;
-    constexpr int PMAX = kV.pmax;
-    static_assert(T - kSymMaxThreshold > WG * PMAX + 1, "table must keep room for in-flight inserts");
-    using Meta = ChunkMeta<V, EC, false>;
-    __shared__ __align__(16) int tab[T];
-    __shared__ Meta cm;
-    __shared__ int s_tmp[WG / kWave];
-    __shared__ int s_n;
+    __shared__ __align__(16) int smem[sym_unit_lds<kSymMaxVariant>() / 4];
     const int2* bin_items = items + static_cast<long long>(bin) * bin_cap;
-    const int count = meta->sym_count[bin].v;
+    const int count = meta->sym_count[bin].v + meta->over_count.v;
     for (int u = blockIdx.x; u < count; u += gridDim.x) {
-        lds_fill<T, WG>(tab, kEmpty, threadIdx.x);
-        if (threadIdx.x == 0) s_n = 0;
-        __syncthreads();
         const int2 it = bin_items[u];
-        const GProb<V> P = ps.get(it.x);
-        const int a0 = P.a_rpt[it.y];
-        const int a1 = P.a_rpt[it.y + 1];
-        bool over = false;
-        for (int ebase = a0; ebase < a1 && !over; ebase += EC) {
-            int start[EC / WG];
-            const int total = load_chunk<V, WG, EC, false>(P, ebase, a1, threadIdx.x, &cm, s_tmp, start);
-            int prior = 0;
-            for (int base = 0; base < total && !over; base += WG * PMAX) {
-                int key[PMAX];
-                V prod[PMAX];
-                bool ok[PMAX];
-                fetch_products<V, WG, EC, PMAX, false>(P, &cm, total, base, threadIdx.x, start, prior, key, prod,
-                                                       ok);
-                const int mine = table_insert_all<T>(tab, key, ok);
-                if (mine) atomicAdd(&s_n, mine);
-                __syncthreads();
-                over = s_n > kSymMaxThreshold;  // uniform: every lane reads after the barrier
-                __syncthreads();
-            }
-        }
+        const GProb<V> P = ps.get(uniform(it.x));
+        const int row = uniform(it.y);
+        const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kSymMaxThreshold>(P, row, smem);
         if (threadIdx.x == 0) {
-            const int n = s_n;
             if (n <= kSymMaxThreshold) {
-                P.c_rpt[it.y] = n;
+                P.c_rpt[row] = n;
             } else {
                 const int f = atomicAdd(&meta->fail_count.v, 1);
                 fail_items[f] = it;
-                fail_off[f] = static_cast<long long>(atomicAdd(
-                    &meta->fail_pool.v, static_cast<unsigned long long>(global_table_slots(P.nip[it.y]))));
+                fail_off[f] = static_cast<long long>(
+                    atomicAdd(&meta->fail_pool.v, static_cast<unsigned long long>(global_table_slots(P.nip[row]))));
             }
         }
-        __syncthreads();
     }
 }
 
@@ -239,23 +310,14 @@ __global__ __launch_bounds__(1024) void k_sym_global(ProbSet<V> ps, const int2* 
 // ----------------------------------------------------------------- launchers
 
 template <typename V>
-void launch_sym_multi(int part, const ProbSet<V>& ps, const int2* items, int bin_cap, const BinTable& sym,
-                      int n_multi, const DevMeta* meta, int grid, hipStream_t s) {
-    if (part == 0)
-        hipLaunchKernelGGL((k_sym_multi<V, kSymPartLo[0], kSymPartHi[0]>), dim3(grid), dim3(kMultiThreads), 0, s, ps,
-                           items, bin_cap, sym, n_multi, meta);
-    else if (part == 1)
-        hipLaunchKernelGGL((k_sym_multi<V, kSymPartLo[1], kSymPartHi[1]>), dim3(grid), dim3(kMultiThreads), 0, s, ps,
-                           items, bin_cap, sym, n_multi, meta);
-    else
-        hipLaunchKernelGGL((k_sym_multi<V, kSymPartLo[2], kSymPartHi[2]>), dim3(grid), dim3(kMultiThreads), 0, s, ps,
-                           items, bin_cap, sym, n_multi, meta);
+void launch_sym_multi(const ProbSet<V>& ps, int2* items, int bin_cap, const BinTable& sym, int n_multi, DevMeta* meta,
+                      int grid, hipStream_t s) {
+    hipLaunchKernelGGL(k_sym_multi<V>, dim3(grid), dim3(kMultiThreads), 0, s, ps, items, bin_cap, sym, n_multi, meta);
 }
 
 template <typename V>
-void launch_sym_max(const ProbSet<V>& ps, const int2* items, int bin_cap, const BinTable& sym, int bin,
-                    DevMeta* meta, int2* fail_items, long long* fail_off, int grid, hipStream_t s) {
-    (void)sym;
+void launch_sym_max(const ProbSet<V>& ps, const int2* items, int bin_cap, int bin, DevMeta* meta, int2* fail_items,
+                    long long* fail_off, int grid, hipStream_t s) {
     hipLaunchKernelGGL(k_sym_max<V>, dim3(grid), dim3(1024), 0, s, ps, items, bin_cap, bin, meta, fail_items,
                        fail_off);
 }
@@ -267,16 +329,9 @@ void launch_sym_global(const ProbSet<V>& ps, const int2* fail_items, const long 
 }
 
 template <typename V>
-int occupancy_sym_multi(int part) {
+int occupancy_sym_multi() {
     int n = 0;
-    const hipError_t e =
-        part == 0   ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                          &n, k_sym_multi<V, kSymPartLo[0], kSymPartHi[0]>, kMultiThreads, 0)
-        : part == 1 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                          &n, k_sym_multi<V, kSymPartLo[1], kSymPartHi[1]>, kMultiThreads, 0)
-                    : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                          &n, k_sym_multi<V, kSymPartLo[2], kSymPartHi[2]>, kMultiThreads, 0);
-    if (e != hipSuccess) n = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_sym_multi<V>, kMultiThreads, 0) != hipSuccess) n = 1;
     return n > 0 ? n : 1;
 }
 
@@ -287,14 +342,14 @@ int occupancy_sym_max() {
     return n > 0 ? n : 1;
 }
 
-#define SPG_INSTANTIATE_SYM(V)                                                                           \
-    template void launch_sym_multi<V>(int, const ProbSet<V>&, const int2*, int, const BinTable&, int,      \
-                                      const DevMeta*, int, hipStream_t);                                  \
-    template void launch_sym_max<V>(const ProbSet<V>&, const int2*, int, const BinTable&, int, DevMeta*,   \
-                                    int2*, long long*, int, hipStream_t);                                 \
-    template void launch_sym_global<V>(const ProbSet<V>&, const int2*, const long long*, int*, int,        \
-                                       hipStream_t);                                                      \
-    template int occupancy_sym_multi<V>(int);                                                             \
+#define SPG_INSTANTIATE_SYM(V)                                                                               \
+    template void launch_sym_multi<V>(const ProbSet<V>&, int2*, int, const BinTable&, int, DevMeta*, int,     \
+                                      hipStream_t);                                                          \
+    template void launch_sym_max<V>(const ProbSet<V>&, const int2*, int, int, DevMeta*, int2*, long long*, int, \
+                                    hipStream_t);                                                            \
+    template void launch_sym_global<V>(const ProbSet<V>&, const int2*, const long long*, int*, int,           \
+                                       hipStream_t);                                                         \
+    template int occupancy_sym_multi<V>();                                                                   \
     template int occupancy_sym_max<V>();
 
 SPG_INSTANTIATE_SYM(float)

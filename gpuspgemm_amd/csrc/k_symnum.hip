@@ -208,7 +208,8 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
     wave_products<V, N, true>(W, uniform(it.a0), uniform(it.a1), &row.walk,
                               [&](const int(&key)[N], const LdsSum(&prod)[N], const bool(&ok)[N]) {
                                   uint32_t h[N];
-                                  table_slots<T>(row.keys, key, ok, h);
+                                  int fresh = 0;
+                                  table_slots<T>(row.keys, key, ok, h, fresh);
 #pragma unroll
                                   for (int j = 0; j < N; ++j)
                                       if (ok[j]) lds_add(row.vals + h[j], prod[j]);
@@ -259,7 +260,7 @@ template <typename V, int VV>
 __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem* __restrict__ items, int first,
                                             int end, int* smem, int* s_tmp, DevMeta* meta) {
     constexpr NumVariant kV = kNumVariants[VV];
-    if constexpr (num_wave_row(kV)) {
+    if constexpr (num_is_wave(kV)) {
         const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
         if (first + wave < end)
             symnum_wave_row<V, kV.p, kV.t, kV.pmax>(ps, items, first + wave,

@@ -197,6 +197,7 @@ struct alignas(128) Counter {
 // when overflowed rows force that stage to run twice.
 struct DevMeta {
     Counter<int32_t> sym_count[kMaxBins];
+    Counter<int32_t> over_count;  // rows added to the last symbolic bin's list by its overflowing neighbour
     Counter<int32_t> fail_count;
     Counter<int32_t> flags;
     Counter<int32_t> max_nip;

@@ -21,34 +21,38 @@ struct NumVariant {
     int t;                   // table slots of the one-wave rows
 };
 // Rows of one wave each (wg / r == 64): see symnum_wave_row.
-constexpr bool num_wave_row(const NumVariant& v) { return v.wg / v.r == kWave; }
+constexpr bool num_is_wave(const NumVariant& v) { return v.wg / v.r == kWave; }
 
 
-// Symbolic (count) variants.  0..8 run inside one multi-bin launch of 256
-// threads; 9 is the largest LDS table with overflow detection
-// (sym1.cuh:169-245).  A bin may take rows of NIP below the table size.
+// Symbolic (count) variants.  0..8 run inside one launch of 256-thread
+// workgroups: 0..4 several rows to a wave, 5 and 6 a row to a wave, 7 and 8 a
+// row to a workgroup; 9 is the largest LDS table (sym1.cuh:169-245).  A bin
+// may take rows of NIP below its table size; variant 8 takes rows of any NIP
+// and hands those with more than kSymOverThreshold distinct columns to
+// variant 9, which hands those above kSymMaxThreshold to the global tables.
+// A row's NIP says little about its distinct columns: a structural matrix of
+// 81 entries a row has 6,561 products and 375 columns, and a 1024-thread
+// workgroup with a 128 KB table per such row took 1.54 ms for 59,049 rows.
 constexpr SymVariant kSymVariants[] = {
     {256, 256, 16, 4, 8},  {256, 128, 32, 4, 8},  {256, 64, 64, 8, 8},    {256, 32, 128, 16, 8},
-    {256, 16, 256, 32, 8}, {256, 4, 512, 64, 8},  {256, 4, 1024, 64, 12}, {256, 1, 4096, 256, 8},
-    {256, 1, 8192, 256, 8}, {1024, 1, 32768, 1024, 4},
+    {256, 16, 256, 32, 8}, {256, 4, 512, 64, 4},  {256, 4, 1024, 64, 4},  {256, 1, 4096, 64, 4},
+    {256, 1, 4096, 64, 4}, {1024, 1, 32768, 64, 4},
 };
 constexpr int kSymMultiVariants = 9;
+constexpr int kSymOverVariant = 8;
 constexpr int kSymMaxVariant = 9;
-constexpr int kSymMaxThreshold = 26214;  // distinct keys admitted in the 32768-slot table (80 %)
-constexpr int kSymMultiLds = 36 * 1024;  // bytes: max over variants 0..8 of r * sym_row_ints * 4
-// The multi-bin variants run in three launches ("parts"), each with the
-// register and LDS budget of its own variants: small tables (0..3), mid
-// tables (4..6) and the two largest tables (7, 8; a row per workgroup).
-// A launch's LDS is its largest variant's, so keeping the 8192-slot table
-// apart lets the mid tables (the 96^3 stencil's rows) run at 6 waves per
-// SIMD instead of 4 (80 VGPRs, 8 bytes spilled per lane; measured faster
-// than 5 waves without a spill).  kSymMultiMinWaves is each part's
-// residency floor, as for kNumMinWaves.
-constexpr int kSymParts = 3;
-constexpr int kSymPartLo[kSymParts] = {0, 4, 7};
-constexpr int kSymPartHi[kSymParts] = {4, 7, 9};
-constexpr int kSymMultiMinWaves[kSymParts] = {7, 6, 4};
-constexpr int sym_part(int variant) { return variant < kSymPartHi[0] ? 0 : (variant < kSymPartHi[1] ? 1 : 2); }
+// Distinct columns at which a wave of these variants stops inserting; every
+// wave may have a round of 64 * 4 more in flight.  Linear probing gets slow
+// as a table fills: with 70 % here a row that overflowed (95 % with the
+// rounds in flight) took 200 us, with 50 % under 20.
+constexpr int kSymOverThreshold = 2048;  // 50 % of 4096
+constexpr int kSymMaxThreshold = 26214;  // 80 % of 32768
+static_assert(kSymOverThreshold + 4 * 256 < 4096 && kSymMaxThreshold + 16 * 256 < 32768,
+              "a counting table keeps room for the rounds in flight");
+constexpr int kSymMultiLds = 23 * 1024;  // bytes a workgroup of the multi-bin launch may use (seven on a CU)
+constexpr int kSymMultiMinWaves = 7;     // waves per SIMD it keeps: at most 72 VGPRs
+constexpr bool sym_is_wave(const SymVariant& v) { return v.wg / v.r == kWave; }
+constexpr bool sym_is_group(const SymVariant& v) { return v.wg / v.r > kWave; }
 
 // Fused sorted-columns + numeric variants, one kernel each: all use 256
 // threads except 9 (a 1024-thread workgroup per row); rows above every
@@ -123,11 +127,13 @@ constexpr int padded_row_ints(int bytes) {
 // Fused variant: table 2p ints (reused for p sums in double), sorted
 // list p ints, chunk metadata when the row has more than one lane.
 constexpr int num_row_ints(const NumVariant& v) {
-    return num_wave_row(v) ? wave_row_bytes(v.p, v.t) / 4
+    return num_is_wave(v) ? wave_row_bytes(v.p, v.t) / 4
                            : padded_row_ints(12 * v.p + (v.wg / v.r > 1 ? 16 * v.ec : 0));
 }
-// Symbolic variant: table t ints, chunk metadata without values.
+// Symbolic variant: table t ints, walk metadata without values.
 constexpr int sym_row_ints(const SymVariant& v) {
+    if (sym_is_group(v)) return v.t + v.wg / kWave * static_cast<int>(sizeof(WaveChunk<false>)) / 4 + 4;
+    if (sym_is_wave(v)) return v.t + static_cast<int>(sizeof(WaveChunk<false>)) / 4;
     return padded_row_ints(4 * v.t + (v.wg / v.r > 1 ? 8 * v.ec + 8 : 0));
 }
 constexpr int max_sym_multi_lds() {
@@ -186,14 +192,14 @@ void launch_scan_apply(const ProbSet<V>& ps, const BinTable& num, DevMeta* meta,
                        RowItem* items, long long* gpool_off, long long* inst_nnz, int after_fail,
                        int tile_prefix_min, hipStream_t s);
 
-// symbolic count: multi-bin launch over bins [0, n_multi) of `sym`
-// part p: variants [kSymPartLo[p], kSymPartHi[p])
+// symbolic count: one launch over bins [0, n_multi) of `sym` (rows that
+// overflow variant 8 join the list of the last bin), then the last bin
 template <typename V>
-void launch_sym_multi(int part, const ProbSet<V>& ps, const int2* items, int bin_cap, const BinTable& sym,
-                      int n_multi, const DevMeta* meta, int grid, hipStream_t s);
+void launch_sym_multi(const ProbSet<V>& ps, int2* items, int bin_cap, const BinTable& sym, int n_multi, DevMeta* meta,
+                      int grid, hipStream_t s);
 template <typename V>
-void launch_sym_max(const ProbSet<V>& ps, const int2* items, int bin_cap, const BinTable& sym, int bin,
-                    DevMeta* meta, int2* fail_items, long long* fail_off, int grid, hipStream_t s);
+void launch_sym_max(const ProbSet<V>& ps, const int2* items, int bin_cap, int bin, DevMeta* meta, int2* fail_items,
+                    long long* fail_off, int grid, hipStream_t s);
 template <typename V>
 void launch_sym_global(const ProbSet<V>& ps, const int2* fail_items, const long long* fail_off, int* pool,
                        int count, hipStream_t s);
@@ -213,7 +219,7 @@ void launch_symnum_global(const ProbSet<V>& ps, const RowItem* items, const long
 
 // occupancy (workgroups per CU) of the persistent launches
 template <typename V>
-int occupancy_sym_multi(int part);
+int occupancy_sym_multi();
 template <typename V>
 int occupancy_sym_max();
 template <typename V>

@@ -74,8 +74,10 @@ __device__ __forceinline__ uint32_t slot24(int key) {
 // together, each a compare-and-swap; the lanes still probing are kept as
 // scalar masks, so that a key whose lanes are all done costs nothing more.
 // The table never fills (its row has fewer distinct columns than T).
-template <int T, int N>
-__device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const bool (&ok)[N], uint32_t (&h)[N]) {
+// With COUNT, `fresh` grows by the number of keys the wave inserted.
+template <int T, int N, bool COUNT = false>
+__device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const bool (&ok)[N], uint32_t (&h)[N],
+                                            int& fresh) {
     int old[N];
     unsigned long long pend[N];
 #pragma unroll
@@ -87,6 +89,7 @@ __device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         const bool on = ok[j] && old[j] != kEmpty && old[j] != key[j];
+        if constexpr (COUNT) fresh += __popcll(__ballot(ok[j] && old[j] == kEmpty));
         h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
         pend[j] = __ballot(on);
         any |= pend[j];
@@ -99,7 +102,9 @@ __device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             if (!pend[j]) continue;
-            const bool on = in_mask(pend[j]) && old[j] != kEmpty && old[j] != key[j];
+            const bool was = in_mask(pend[j]);
+            const bool on = was && old[j] != kEmpty && old[j] != key[j];
+            if constexpr (COUNT) fresh += __popcll(__ballot(was && old[j] == kEmpty));
             h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
             pend[j] = __ballot(on);
             any |= pend[j];
@@ -261,10 +266,11 @@ struct WaveOperands {
 // number of entries that start at or before it (less one): the chunk's
 // starts are marked in a bitmap, 64 products to a word and one position
 // early, so that a lane counts the marks below its own bit (two mbcnt on
-// top of the count before the word).  `rounds_first` and
-// `rounds_step` let several waves share a row: this wave takes the rounds
-// rounds_first, rounds_first + rounds_step, ... of every chunk, or, with
-// `by_chunk`, every round of the chunks rounds_first, ... instead.
+// top of the count before the word).  `first` and `step` let
+// several waves share a row: this wave takes the rounds first, first + step,
+// ... of every window, or, with `by_chunk`, every round of the chunks first,
+// first + step, ... instead.  An f that
+// returns false (the same on every lane) ends the walk.
 template <typename V, int N, bool VALS, bool WIDE, typename F>
 __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                                  int first, int step, bool by_chunk) {
@@ -351,7 +357,11 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
 #pragma unroll
                     for (int j = 0; j < N; ++j) prod[j] = a[j] * static_cast<LdsSum>(bv[j]);
                 }
-                f(key, prod, ok);
+                if constexpr (std::is_same_v<decltype(f(key, prod, ok)), bool>) {
+                    if (!f(key, prod, ok)) return;
+                } else {
+                    f(key, prod, ok);
+                }
             }
         }
     }
@@ -364,6 +374,14 @@ __device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, 
         wave_products_at<V, N, VALS, true>(W, a0, a1, wc, f, first, step, by_chunk);
     else
         wave_products_at<V, N, VALS, false>(W, a0, a1, wc, f, first, step, by_chunk);
+}
+
+// How the waves of a workgroup share a row: by chunks of 64 entries when
+// every wave gets one and the rows of B are short (a chunk is then a few
+// rounds), otherwise round by round, each wave reading every chunk.
+template <int WAVES>
+__device__ __forceinline__ bool wave_by_chunk(int entries, int nip) {
+    return entries >= WAVES * kWave && nip / 16 < entries;
 }
 
 }  // namespace spg

@@ -342,6 +342,31 @@ def test_wave_rows_windows_and_wide_offsets(emu, tmp_path, variant):
                 call(A.astype(np.float32), B.astype(np.float32), "--f32", tables=table, env={"SPG_WIDE_MIN": "0"}))
 
 
+def test_symbolic_overflow_moves_to_the_largest_table(emu, tmp_path):
+    """Workgroup rows of the variant that takes any NIP: 2,049 to 4,000
+    distinct columns pass its limit and are counted again by the largest
+    table, 2,048 and fewer (one row with 6,000 products on 300 columns)
+    stay; rows of B long enough for the waves to share rounds, and short
+    ones with enough entries of A for them to share chunks."""
+    over = next(v["id"] for v in _SV if v["id"] == SYM_MAX - 1)
+    table = {0: f"{over} 100000 {INT_MAX}\n{SYM_MAX} {INT_MAX} {INT_MAX}\n"}
+
+    def matrix(rows, n, seed):
+        rpt = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+        col = np.concatenate(rows).astype(np.int32)
+        return HostCSR(len(rows), n, rpt, col, gen.rand_unit(seed, 1, np.arange(col.size)) * 2 - 1)
+
+    # long rows of B: row k holds the columns 100 k .. 100 k + 99, the last 60 rows the columns 0 .. 299 in parts
+    wide = [np.arange(100 * k, 100 * k + 100) for k in range(40)]
+    wide += [np.arange(100 * (k % 3), 100 * (k % 3) + 100) for k in range(60)]
+    B = matrix(wide, 4000, 91)
+    A = matrix([np.arange(0, 40), np.arange(0, 20), np.r_[0:20, 20], np.arange(40, 100)], 100, 92)
+    # one entry a row: 2,048, 2,049 and 300 distinct columns
+    B1 = matrix([[k] for k in range(3000)], 3000, 93)
+    A1 = matrix([np.arange(2048), np.arange(2049), np.arange(100, 400)], 3000, 94)
+    run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A1, B1, "--f32", tables=table))
+
+
 def test_global_paths(emu, tmp_path):
     """The heavy-row case first with the default tables and then with every
     row forced to the global kernels."""
