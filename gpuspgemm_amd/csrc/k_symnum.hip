@@ -255,6 +255,123 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
     wave_sync();  // LDS is reused by the next row
 }
 
+// The same for a row of a whole workgroup.  Every wave walks a share of the
+// products on its own and all add into one table.  Each wave then sorts a
+// block of the compacted columns in registers; a column's place in C is its
+// place in its block plus the number of smaller columns in every other block
+// (binary searches in LDS), where it leaves its table slot for the coalesced
+// write of C.  27^3 nodes of 3 unknowns (6,561 products, 375 columns a row,
+// FP64): 1.74 ms for the launch with two walks and a search per product,
+// 0.46 ms so.  Rows up to 512 columns have a variant of their own, whose
+// 18 KB of LDS let eight workgroups share a CU (31 KB for 1024: five).
+template <typename V, int WG, int P, int T, int N>
+__device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const RowItem* __restrict__ items, int idx,
+                                                 GroupRow<P, T, WG / kWave>& row, DevMeta* meta) {
+    constexpr int kWaves = WG / kWave;
+    constexpr int B = P / kWaves;  // columns of a wave's block
+    constexpr int E = B / kWave;
+    constexpr int S = T / WG;
+    const int lane = lane_id();
+    const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+    {
+        typedef int Words __attribute__((vector_size(16)));
+        Words* k = reinterpret_cast<Words*>(row.keys);
+        Words* v = reinterpret_cast<Words*>(row.vals);
+#pragma unroll
+        for (int i = 0; i < T / (4 * WG); ++i) k[i * WG + threadIdx.x] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+#pragma unroll
+        for (int i = 0; i < T / (2 * WG); ++i) v[i * WG + threadIdx.x] = Words{0, 0, 0, 0};
+    }
+    const RowItem it = load_item(items, idx);
+    const GProb<V> Pr = ps.get(uniform(it.inst));
+    const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+    const int a0 = uniform(it.a0), a1 = uniform(it.a1);
+    __syncthreads();
+    wave_products<V, N, true>(
+        W, a0, a1, &row.walk[wave],
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const bool(&ok)[N]) {
+            uint32_t h[N];
+            int fresh = 0;
+            table_slots<T>(row.keys, key, ok, h, fresh);
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                if (ok[j]) lds_add(row.vals + h[j], prod[j]);
+        },
+        wave, kWaves, wave_by_chunk<kWaves>(a1 - a0, uniform(it.nip)));
+    __syncthreads();
+
+    // the occupied slots, S consecutive ones to a thread, in front of each other
+    int key[S];
+    int mine = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        key[s] = row.keys[threadIdx.x * S + s];
+        mine += key[s] != kEmpty ? 1 : 0;
+    }
+    const int incl = wave_incl_scan(mine);
+    if (lane == kWave - 1) row.wave_sum[wave] = incl;
+    __syncthreads();
+    int found = 0, pos = incl - mine;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        const int n = row.wave_sum[w];
+        pos += w < wave ? n : 0;
+        found += n;
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (key[s] != kEmpty) {
+            if (pos < P) row.cols[pos] = key[s];
+            ++pos;
+        }
+    __syncthreads();
+    const int cn = uniform(it.cn);
+    if (threadIdx.x == 0 && cn != found) atomicOr(&meta->flags.v, kFlagMismatch);
+    const int n = min(found, P);
+    const int w = min(n, cn);
+    const int mine0 = wave * B + lane * E;
+    int x[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) x[s] = mine0 + s < n ? row.cols[mine0 + s] : INT_MAX;
+    if (wave * B < n) {
+        wave_sort<E>(x);
+#pragma unroll
+        for (int s = 0; s < E; ++s) row.cols[mine0 + s] = x[s];
+    }
+    __syncthreads();
+    if (wave * B < n) {
+        int rank[E];
+#pragma unroll
+        for (int s = 0; s < E; ++s) rank[s] = lane * E + s;
+#pragma unroll
+        for (int o = 1; o < kWaves; ++o) {
+            const int other = (wave + o) % kWaves;
+            if (other * B >= n) continue;
+            int at[E];
+            lower_bound_all<B, E>(row.cols + other * B, x, at);
+#pragma unroll
+            for (int s = 0; s < E; ++s) {
+                // (a block of B columns may hold none as large: B steps of the search end one short)
+                at[s] += row.cols[other * B + at[s]] < x[s] ? 1 : 0;
+                rank[s] += at[s];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < E; ++s)
+            if (mine0 + s < n) row.slots[rank[s]] = static_cast<unsigned short>(table_find<T>(row.keys, x[s]));
+    }
+    __syncthreads();
+    const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);
+    const auto cval = uniform_ptr(Pr.c_val) + uniform(it.c0);
+    for (int j = threadIdx.x; j < w; j += WG) {
+        const int h = row.slots[j];
+        ccol[j] = row.keys[h];
+        cval[j] = static_cast<V>(row.vals[h]);
+    }
+    __syncthreads();  // LDS is reused by the next row
+}
+
 // The rows [first, end) of one unit of variant VV.
 template <typename V, int VV>
 __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem* __restrict__ items, int first,
@@ -265,6 +382,9 @@ __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem*
         if (first + wave < end)
             symnum_wave_row<V, kV.p, kV.t, kV.pmax>(ps, items, first + wave,
                                                     reinterpret_cast<WaveRow<kV.p, kV.t>*>(smem)[wave], meta);
+    } else if constexpr (num_is_group(kV)) {
+        symnum_group_row<V, kV.wg, kV.p, kV.t, kV.pmax>(
+            ps, items, first, *reinterpret_cast<GroupRow<kV.p, kV.t, kV.wg / kWave>*>(smem), meta);
     } else {
         symnum_rows<V, kV.wg, kV.r, kV.p, kV.ec, kV.pmax>(ps, items, first, end, smem, s_tmp, meta);
     }
@@ -287,7 +407,7 @@ __global__ __launch_bounds__(kNumVariants[VV].wg) SPG_WAVES_PER_EU(kNumMinWaves[
 }
 
 #define SPG_NUM_VARIANTS(X) \
-    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18)
+    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19)
 
 // Several bins of the fused pass in one launch, a workgroup per unit.
 // Each XCD gets a contiguous slice of every bin (balanced work across the

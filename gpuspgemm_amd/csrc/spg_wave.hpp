@@ -250,6 +250,31 @@ static_assert(sizeof(WaveRow<128, 256>) == wave_row_bytes(128, 256) &&
                   sizeof(WaveRow<512, 1024>) == wave_row_bytes(512, 1024),
               "LDS size of a wave's row");
 
+// The same for a row that WAVES waves share: the compacted columns, then the
+// table slots of the row's columns in ascending order.
+template <int P, int T, int WAVES>
+struct alignas(16) GroupRow {
+    LdsSum vals[T];
+    int keys[T];
+    union {
+        WaveChunk<true> walk[WAVES];
+        struct {
+            int cols[P];
+            unsigned short slots[P];
+        };
+    };
+    int wave_sum[WAVES];
+};
+constexpr int group_row_bytes(int p, int t, int waves) {
+    const int walk = waves * static_cast<int>(sizeof(WaveChunk<true>));
+    const int sorted = 6 * p;
+    const int all = t * static_cast<int>(sizeof(LdsSum) + sizeof(int)) + (walk > sorted ? walk : sorted) + 4 * waves;
+    return (all + 15) / 16 * 16;
+}
+static_assert(sizeof(GroupRow<512, 1024, 4>) == group_row_bytes(512, 1024, 4) &&
+                  sizeof(GroupRow<1024, 2048, 4>) == group_row_bytes(1024, 2048, 4),
+              "LDS size of a workgroup's row");
+
 // Where a wave's walk reads (all scalar).
 template <typename V>
 struct WaveOperands {
