@@ -60,6 +60,7 @@ template <typename V, int T, int N>
 __device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* __restrict__ items, int idx, int step,
                                               int end, int* smem) {
     typedef int Words __attribute__((vector_size(16)));
+    static_assert(T % (4 * kWave) == 0, "every lane clears a whole share");
     const int lane = lane_id();
     int* tab = smem;
     auto* walk = reinterpret_cast<WaveChunk<false>*>(smem + T);
@@ -104,6 +105,7 @@ template <typename V, int WG, int T, int N, int LIMIT>
 __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* smem) {
     typedef int Words __attribute__((vector_size(16)));
     constexpr int kWaves = WG / kWave;
+    static_assert(T % (4 * WG) == 0, "every thread clears a whole share");
     const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
     int* tab = smem;
     auto* walk = reinterpret_cast<WaveChunk<false>*>(smem + T);

@@ -75,6 +75,145 @@ __device__ __forceinline__ int sort_row(const int* tab, int* cols, int lr, int* 
     return found;
 }
 
+// Rows of at most L * K products, a group of L lanes to a row (K = 1, or L =
+// 64), when the whole wave's rows are such: sorted in registers instead of
+// hashed.  A row's products take one slot each, product j * 64 + lane of the
+// wave; the slots' entries come from a bitmap of entry starts as in
+// wave_products.  Every slot packs its column above its slot number into one
+// word, the groups sort the words, a slot whose column differs from the one
+// below starts an entry of C, and its place in the row is the number of such
+// slots before it.  No table, no probing, and LDS sums only for waves that
+// have a repeated column.  Bound by VALU issue (about 100 instructions for
+// the 8 rows of a wave at L = 8, where the hashed path spends 25 a row).
+template <int K>
+struct alignas(16) SortSlots {
+    unsigned long long starts[K];
+    union {
+        WaveEntry<true> ent[kWave];
+        LdsSum prod[kWave * K];
+    };
+    LdsSum sum[kWave * K];
+};
+template <int K>
+constexpr int kSortColBits = K == 1 ? 26 : 25;  // column bits beside the slot number (all ones: no product)
+
+template <typename V, int L, int K>
+__device__ __forceinline__ void symnum_sorted(const GProb<V>& Pr, const RowItem& it, bool active, SortSlots<K>& sl,
+                                              DevMeta* meta) {
+    static_assert(K == 1 || (K == 2 && L == kWave), "slot order");
+    constexpr int kSlotBits = K == 1 ? 6 : 7;
+    const int lane = lane_id();
+    const int lr = lane % L;
+    const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
+                            uniform_ptr(Pr.b_val), false};
+    const auto c_col = uniform_ptr(Pr.c_col);
+    const auto c_val = uniform_ptr(Pr.c_val);
+    if (lane < K) sl.starts[lane] = 0;
+    const int nip = active ? it.nip : 0;
+    // an entry of A to a lane
+    long long ref = 0;
+    V av = V(0);
+    if (active && it.a0 + lr < it.a1) {
+        ref = W.bref[it.a0 + lr];
+        av = W.a_val[it.a0 + lr];
+    }
+    const int len = bref_len(ref);
+    const int start = group_excl_sum<L>(len);
+    wave_sync();
+    if (len > 0) {
+        const int at = lane - lr + start;  // the slot of the entry's first product
+        atomicOr(&sl.starts[K == 1 ? 0 : at >> 6], 1ull << (at & 63));
+    }
+    const unsigned long long filled = __ballot(len > 0);
+    if (len > 0) {
+        WaveEntry<true> w;
+        w.av = av;
+        w.d = (bref_start(ref) - start) * 4;  // bytes of b_col, modulo 2^32
+        sl.ent[rank_in(filled)] = w;
+    }
+    wave_sync();
+    uint32_t word[K];
+    LdsSum prod[K];
+    int before = -1;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const unsigned long long m = sl.starts[j];
+        const unsigned lo = static_cast<unsigned>(uniform(static_cast<int>(m)));
+        const unsigned hi = static_cast<unsigned>(uniform(static_cast<int>(m >> 32)));
+        const unsigned long long mu = static_cast<unsigned long long>(hi) << 32 | lo;
+        const int e = before + rank_in(mu) + (in_mask(mu) ? 1 : 0);
+        before += __popcll(mu);
+        const bool ok = j * kWave + lr < nip;
+        const WaveEntry<true> w = sl.ent[ok ? e : 0];
+        const uint32_t pos = static_cast<uint32_t>(w.d) + static_cast<uint32_t>((j * kWave + lr) * 4);
+        const uint32_t o = ok ? pos : 0u;
+        const int key = *(const int32_t SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_col + o);
+        const V bv = *(const V SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_val + o * static_cast<uint32_t>(sizeof(V) / 4));
+        prod[j] = w.av * static_cast<LdsSum>(bv);
+        word[j] = ok ? static_cast<uint32_t>(key) << kSlotBits | static_cast<uint32_t>(j * kWave + lane) : ~0u;
+    }
+    wave_sync();  // every lane has read its entries
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        sl.prod[j * kWave + lane] = prod[j];
+        sl.sum[j * kWave + lane] = 0;
+    }
+    wave_sort<K, L>(word);
+    wave_sync();
+    // sorted slot lane * K + s of the wave; heads: first of its column in its row
+    uint32_t below = lane_below(word[K - 1]);
+    bool head[K], real[K];
+    unsigned long long heads[K], repeats = 0;
+    const unsigned long long group = L == kWave ? ~0ull : ((1ull << (L % kWave)) - 1) << (lane - lr);
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+        real[s] = word[s] != ~0u;
+        head[s] = real[s] && ((s == 0 && lr == 0) || (word[s] >> kSlotBits) != (below >> kSlotBits));
+        heads[s] = __ballot(head[s]);
+        repeats |= __ballot(real[s] && !head[s]);
+        below = word[s];
+    }
+    int rank[K];
+    int found = 0;
+#pragma unroll
+    for (int s = 0; s < K; ++s) found += __popcll(heads[s] & group);
+#pragma unroll
+    for (int s = 0; s < K; ++s) {
+        rank[s] = 0;
+#pragma unroll
+        for (int t = 0; t < K; ++t) rank[s] += rank_in(heads[t] & group) + (t < s && head[t] ? 1 : 0);
+    }
+    if (active && lr == 0 && found != it.cn) atomicOr(&meta->flags.v, kFlagMismatch);
+    LdsSum val[K];
+#pragma unroll
+    for (int s = 0; s < K; ++s) val[s] = sl.prod[word[s] & (kWave * K - 1)];
+    if (repeats) {
+        const int g0 = (lane - lr) * K;  // the row's first place among the sums
+#pragma unroll
+        for (int s = 0; s < K; ++s)
+            if (real[s]) lds_add(&sl.sum[g0 + rank[s] - (head[s] ? 0 : 1)], val[s]);
+        wave_sync();
+#pragma unroll
+        for (int s = 0; s < K; ++s)
+            if (head[s]) val[s] = sl.sum[g0 + rank[s]];
+    }
+#pragma unroll
+    for (int s = 0; s < K; ++s)
+        if (head[s] && rank[s] < it.cn) {
+            c_col[it.c0 + rank[s]] = static_cast<int32_t>(word[s] >> kSlotBits);
+            c_val[it.c0 + rank[s]] = static_cast<V>(val[s]);
+        }
+    wave_sync();  // LDS is reused by the next rows
+}
+
+// Whether symnum_sorted takes a wave's rows (every lane: its row's item).
+template <typename V, int L, int K>
+__device__ __forceinline__ bool sorted_fits(const GProb<V>& Pr, const RowItem& it, bool active) {
+    const bool fits = it.nip <= L * K && it.a1 - it.a0 <= L && it.inst == uniform(it.inst) && !Pr.wide &&
+                      Pr.n < 1 << kSortColBits<K>;
+    return __ballot(active && !fits) == 0;
+}
+
 template <typename V, int WG, int R, int P, int EC, int PMAX>
 __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem* __restrict__ items, int first,
                                             int end, int* smem, int* s_tmp, DevMeta* meta) {
@@ -94,12 +233,21 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     Meta* cm = reinterpret_cast<Meta*>(cols + P);
     LdsSum* vals = reinterpret_cast<LdsSum*>(tab);
 
-    lds_fill<T, L>(tab, kEmpty, lr);
-    gsync<L>();
-
     const int idx = first + slot;
     const bool active = idx < end;
     const RowItem it = active ? load_item(items, idx) : RowItem{0, 0, 0, 0, 0, 0, 0, 0};
+    if constexpr (L >= 8 && L < kWave && P == L) {
+        const GProb<V> Pu = ps.get(uniform(it.inst));
+        if (sorted_fits<V, L, 1>(Pu, it, active)) {
+            static_assert(kWave / L * ROW_INTS * 4 >= static_cast<int>(sizeof(SortSlots<1>)) &&
+                              kWave / L * ROW_INTS % 4 == 0, "a wave's slots lie in its rows' LDS");
+            symnum_sorted<V, L, 1>(Pu, it, active, *reinterpret_cast<SortSlots<1>*>(tab - slot % (kWave / L) * ROW_INTS),
+                                   meta);
+            return;
+        }
+    }
+    lds_fill<T, L>(tab, kEmpty, lr);
+    gsync<L>();
     const GProb<V> Pr = ps.get(it.inst);
     const int a0 = it.a0, a1 = it.a1, nip = it.nip, c0 = it.c0, cn = it.cn;
     // products staged in registers when the whole row fits in one round
@@ -189,19 +337,26 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
                                                 WaveRow<P, T>& row, DevMeta* meta) {
     constexpr int E = P / kWave;
     constexpr int S = T / kWave;
+    static_assert(T % (2 * kWave) == 0 && P % kWave == 0, "every lane clears and compacts whole shares");
     const int lane = lane_id();
+    const RowItem it = load_item(items, idx);
+    const GProb<V> Pr = ps.get(uniform(it.inst));
+    if constexpr (P <= 2 * kWave) {
+        if (sorted_fits<V, kWave, P / kWave>(Pr, it, true)) {
+            symnum_sorted<V, kWave, P / kWave>(Pr, it, true, *reinterpret_cast<SortSlots<P / kWave>*>(&row), meta);
+            return;
+        }
+    }
     {
         typedef int Words __attribute__((vector_size(16)));
         Words* k = reinterpret_cast<Words*>(row.keys);
         Words* v = reinterpret_cast<Words*>(row.vals);
 #pragma unroll
-        for (int i = 0; i < T / (4 * kWave); ++i) k[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+        for (int i = lane; i < T / 4; i += kWave) k[i] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
 #pragma unroll
         for (int i = 0; i < T * static_cast<int>(sizeof(LdsSum)) / (16 * kWave); ++i)
             v[i * kWave + lane] = Words{0, 0, 0, 0};
     }
-    const RowItem it = load_item(items, idx);
-    const GProb<V> Pr = ps.get(uniform(it.inst));
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
                             uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
     wave_sync();
@@ -271,6 +426,7 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     constexpr int B = P / kWaves;  // columns of a wave's block
     constexpr int E = B / kWave;
     constexpr int S = T / WG;
+    static_assert(T % (4 * WG) == 0 && P % WG == 0, "every thread clears and compacts whole shares");
     const int lane = lane_id();
     const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
     {

@@ -148,7 +148,7 @@ constexpr unsigned long long larger_lanes(int s) {
     }
     return m;
 }
-// Lanes whose in-lane pair is ascending at level K.
+// Lanes whose in-lane pair falls at level K.
 template <int E, int K>
 constexpr unsigned long long falling_lanes(int s) {
     unsigned long long m = 0;
@@ -157,12 +157,12 @@ constexpr unsigned long long falling_lanes(int s) {
     return m;
 }
 
-template <int E, int K, int J>
-__device__ __forceinline__ void wave_sort_stage(int (&x)[E]) {
+template <int E, int K, int J, typename X>
+__device__ __forceinline__ void wave_sort_stage(X (&x)[E]) {
     if constexpr (J >= E) {
-        int other[E];
+        X other[E];
 #pragma unroll
-        for (int s = 0; s < E; ++s) other[s] = wave_xor<J / E>(x[s]);
+        for (int s = 0; s < E; ++s) other[s] = static_cast<X>(wave_xor<J / E>(static_cast<int>(x[s])));
         static_for<0, E>([&](auto si) {
             constexpr int s = decltype(si)::value;
             constexpr unsigned long long kLarger = larger_lanes<E, K, J>(s);
@@ -172,34 +172,69 @@ __device__ __forceinline__ void wave_sort_stage(int (&x)[E]) {
         static_for<0, E>([&](auto si) {
             constexpr int s = decltype(si)::value;
             if constexpr ((s & J) == 0) {
-                if constexpr (K < E) {  // the direction is the same for every lane
-                    const int lo = min(x[s], x[s + J]), hi = max(x[s], x[s + J]);
-                    x[s] = (s & K) == 0 ? lo : hi;
-                    x[s + J] = (s & K) == 0 ? hi : lo;
-                } else {
-                    constexpr unsigned long long kFalling = falling_lanes<E, K>(s);
-                    const bool keep = (x[s] < x[s + J]) != in_mask(kFalling);
-                    const int a = x[s], b = x[s + J];
-                    x[s] = keep ? a : b;
-                    x[s + J] = keep ? b : a;
-                }
+                const X a = x[s], b = x[s + J];
+                bool keep = a < b;
+                if constexpr (K < E)  // the direction is the same for every lane
+                    keep = keep != ((s & K) != 0);
+                else
+                    keep = keep != in_mask(falling_lanes<E, K>(s));
+                x[s] = keep ? a : b;
+                x[s + J] = keep ? b : a;
             }
         });
     }
 }
-template <int E, int K, int J>
-__device__ __forceinline__ void wave_sort_level(int (&x)[E]) {
+template <int E, int K, int J, typename X>
+__device__ __forceinline__ void wave_sort_level(X (&x)[E]) {
     if constexpr (J >= 1) {
         wave_sort_stage<E, K, J>(x);
         wave_sort_level<E, K, J / 2>(x);
     }
 }
-template <int E, int K = 2>
-__device__ __forceinline__ void wave_sort(int (&x)[E]) {
-    if constexpr (K <= kWave * E) {
+// The last level of a sort: ascending in every group (the level's direction
+// bit lies above every index).
+template <int E, int J, typename X>
+__device__ __forceinline__ void wave_sort_last(X (&x)[E]) {
+    wave_sort_level<E, 2 * kWave * E, J>(x);
+}
+// Every aligned group of L lanes sorts its L * E keys.
+template <int E, int L = kWave, int K = 2, typename X = int>
+__device__ __forceinline__ void wave_sort(X (&x)[E]) {
+    if constexpr (K < L * E) {
         wave_sort_level<E, K, K / 2>(x);
-        wave_sort<E, 2 * K>(x);
+        wave_sort<E, L, 2 * K>(x);
+    } else if constexpr (K == L * E) {
+        wave_sort_last<E, K / 2>(x);
     }
+}
+
+// The value of the lane below (lane 0: its own).
+__device__ __forceinline__ unsigned lane_below(unsigned v) {
+    return static_cast<unsigned>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), 0x138, 0xF, 0xF,
+                                                             false));  // wave_shr:1
+}
+
+// Exclusive prefix sum over aligned groups of L lanes (8 <= L <= 64).
+template <int L>
+__device__ __forceinline__ int group_excl_sum(int v) {
+    static_assert(L == 8 || L == 16 || L == 32 || L == 64, "bad group");
+    int x = v;
+    if constexpr (L == 8) {
+        // row_shr:1 and :2 without the lanes that would read the group below
+        const int a = __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);
+        x += in_mask(0xFEFEFEFEFEFEFEFEull) ? a : 0;
+        const int b = __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);
+        x += in_mask(0xFCFCFCFCFCFCFCFCull) ? b : 0;
+        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xA, false);  // row_shr:4 into banks 1 and 3
+    } else {
+        x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);
+        x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);
+        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);
+        x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);
+        if constexpr (L >= 32) x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);
+        if constexpr (L >= 64) x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
+    }
+    return x - v;
 }
 
 // An entry of A as the wave's lanes read it: a_ik and where its row of B

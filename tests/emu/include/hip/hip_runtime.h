@@ -137,11 +137,12 @@ inline T __shfl_xor(T v, int mask, int width = 64) {
     return emu_shfl_any(v, idx);
 }
 // DPP controls the library uses: quad permutations (lane ^ 1 and lane ^ 2
-// within each quad), row_shr:n and row_ror:n within rows of 16 lanes, and
-// the broadcasts of lane 15 of a row to the next row and of lane 31 to the
-// upper half.  Lanes whose row is masked out, or that read no lane, keep
+// within each quad), row_shr:n and row_ror:n within rows of 16 lanes,
+// wave_shr:1, and the broadcasts of lane 15 of a row to the next row and of lane 31 to the
+// upper half.  Lanes whose row or
+// bank of four is masked out, or that read no lane, keep
 // `old` (0 with bound_ctrl).
-inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int row_mask, int, bool bound_ctrl) {
+inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int row_mask, int bank_mask, bool bound_ctrl) {
     const int self = emu::lane();
     const int row = self >> 4, in_row = self & 15;
     int src = -1;
@@ -151,12 +152,14 @@ inline int __builtin_amdgcn_update_dpp(int old, int v, int ctrl, int row_mask, i
         src = in_row >= (ctrl & 15) ? self - (ctrl & 15) : -1;
     else if (ctrl >= 0x121 && ctrl <= 0x12f)
         src = (row << 4) | ((in_row - (ctrl & 15)) & 15);
+    else if (ctrl == 0x138)  // wave_shr:1
+        src = self - 1;
     else if (ctrl == 0x142)
         src = row > 0 ? (row << 4) - 1 : -1;
     else if (ctrl == 0x143)
         src = self >= 32 ? 31 : -1;
     const int got = emu_shfl_any(v, src < 0 ? self : src);
-    if (!((row_mask >> row) & 1)) return old;
+    if (!((row_mask >> row) & 1) || !((bank_mask >> (in_row >> 2)) & 1)) return old;
     return src >= 0 ? got : (bound_ctrl ? 0 : old);
 }
 inline int __builtin_amdgcn_mov_dpp(int v, int ctrl, int row_mask, int bank_mask, bool bound_ctrl) {

@@ -342,6 +342,40 @@ def test_wave_rows_windows_and_wide_offsets(emu, tmp_path, variant):
                 call(A.astype(np.float32), B.astype(np.float32), "--f32", tables=table, env={"SPG_WIDE_MIN": "0"}))
 
 
+# fused variants that sort rows of at most `products` in registers
+SORTED = [(v, NUM[v][2]) for v in sorted(NUM) if NUM[v][0] == NUM[v][2] or (NUM[v][0] == 64 and NUM[v][2] <= 128)]
+
+
+@pytest.mark.parametrize("variant,products", SORTED)
+@pytest.mark.parametrize("columns", [40, (1 << 25) - 1, 1 << 25, (1 << 26) - 1, 1 << 26])
+def test_sorted_rows(emu, tmp_path, variant, products, columns):
+    """Rows of one product up to the variant's slots and one more (a wave
+    with such a row takes the hashed path), empty rows of B inside them,
+    repeated columns (40 columns), and column counts on both sides of the
+    limit that leaves room for the slot number beside the column."""
+    rng = np.random.default_rng(variant)
+    lens = [0, 1, 2, 3, 5, 7, 1, 4]
+    pool = np.unique(np.r_[0, 1, columns - 1, rng.integers(0, columns, 40)])
+    b_rows = [np.sort(rng.choice(pool, size=min(lens[k % 8], len(pool)), replace=False)) for k in range(64)]
+    a_rows, per_wave = [], max(1, 64 // NUM[variant][0])
+    for total in [products, 1, products - 1, products // 2, products + 1, products, 2, 3]:
+        for _ in range(per_wave):  # a row whose products come close to `total`, in random order of B's rows
+            row, have = [], 0
+            for k in rng.permutation(64):
+                if have + len(b_rows[k]) <= total and len(row) < NUM[variant][0]:
+                    row.append(k)
+                    have += len(b_rows[k])
+            a_rows.append(np.sort(row))
+
+    def matrix(rows, n, seed):
+        rpt = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+        col = np.concatenate(rows).astype(np.int32)
+        return HostCSR(len(rows), n, rpt, col, gen.rand_unit(seed, 1, np.arange(col.size)) * 2 - 1)
+    A, B = matrix(a_rows, 64, 95), matrix(b_rows, columns, 96)
+    table = {1: f"{variant} {INT_MAX} {NUM[variant][2]}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
+    run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A, B, "--f32", tables=table))
+
+
 def test_symbolic_overflow_moves_to_the_largest_table(emu, tmp_path):
     """Workgroup rows of the variant that takes any NIP: 2,049 to 4,000
     distinct columns pass its limit and are counted again by the largest
