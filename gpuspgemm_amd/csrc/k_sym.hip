@@ -81,7 +81,7 @@ __device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* 
         const GProb<V> P_next = ps.get(inst_next);
         const int b0 = P_next.a_rpt[row_next], b1 = P_next.a_rpt[row_next + 1];
         int n = 0;
-        wave_products<V, N, false>(W, a0, a1, walk, [&](const int(&key)[N], const LdsSum(&)[N], const bool(&ok)[N]) {
+        wave_products<V, N, false>(W, a0, a1, walk, [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) {
             uint32_t h[N];
             table_slots<T, N, true>(tab, key, ok, h, n);
         });
@@ -125,7 +125,7 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
     };
     wave_products<V, N, false>(
         W, a0, a1, walk + wave,
-        [&](const int(&key)[N], const LdsSum(&)[N], const bool(&ok)[N]) -> bool {
+        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) -> bool {
             if constexpr (LIMIT > 0) {
                 if (uniform(lds_load(total)) > LIMIT) return false;
             }

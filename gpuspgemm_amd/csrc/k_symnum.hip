@@ -361,17 +361,18 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
                             uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
     wave_sync();
     wave_products<V, N, true>(W, uniform(it.a0), uniform(it.a1), &row.walk,
-                              [&](const int(&key)[N], const LdsSum(&prod)[N], const bool(&ok)[N]) {
+                              [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
                                   uint32_t h[N];
                                   int fresh = 0;
                                   table_slots<T>(row.keys, key, ok, h, fresh);
 #pragma unroll
                                   for (int j = 0; j < N; ++j)
-                                      if (ok[j]) lds_add(row.vals + h[j], prod[j]);
+                                      if (in_mask(ok[j])) lds_add(row.vals + h[j], prod[j]);
                               });
     wave_sync();
 
     // the occupied slots, S consecutive ones to a lane, in front of each other
+    const SlotWord<T> sw(uniform(Pr.n));
     int key[S];
     int mine = 0;
 #pragma unroll
@@ -385,18 +386,18 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
 #pragma unroll
     for (int s = 0; s < S; ++s)
         if (key[s] != kEmpty) {
-            if (pos < P) row.cols[pos] = key[s];
+            if (pos < P) row.words[pos] = sw.pack(key[s], lane * S + s);
             ++pos;
         }
     wave_sync();
     const int cn = uniform(it.cn);
     if (lane == 0 && cn != found) atomicOr(&meta->flags.v, kFlagMismatch);
     const int w = min(min(found, P), cn);
-    int x[E];
+    uint32_t x[E];
 #pragma unroll
     for (int s = 0; s < E; ++s) {
-        x[s] = row.cols[lane * E + s];
-        if (lane * E + s >= found) x[s] = INT_MAX;
+        x[s] = row.words[lane * E + s];
+        if (lane * E + s >= found) x[s] = ~0u;
     }
     wave_sort<E>(x);
     const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);
@@ -404,8 +405,8 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
 #pragma unroll
     for (int s = 0; s < E; ++s)
         if (lane * E + s < w) {
-            ccol[lane * E + s] = x[s];
-            cval[lane * E + s] = static_cast<V>(row.vals[table_find<T>(row.keys, x[s])]);
+            ccol[lane * E + s] = sw.column(x[s]);
+            cval[lane * E + s] = static_cast<V>(row.vals[sw.slot(row.keys, x[s])]);
         }
     wave_sync();  // LDS is reused by the next row
 }
@@ -446,18 +447,19 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     __syncthreads();
     wave_products<V, N, true>(
         W, a0, a1, &row.walk[wave],
-        [&](const int(&key)[N], const LdsSum(&prod)[N], const bool(&ok)[N]) {
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
             uint32_t h[N];
             int fresh = 0;
             table_slots<T>(row.keys, key, ok, h, fresh);
 #pragma unroll
             for (int j = 0; j < N; ++j)
-                if (ok[j]) lds_add(row.vals + h[j], prod[j]);
+                if (in_mask(ok[j])) lds_add(row.vals + h[j], prod[j]);
         },
         wave, kWaves, wave_by_chunk<kWaves>(a1 - a0, uniform(it.nip)));
     __syncthreads();
 
     // the occupied slots, S consecutive ones to a thread, in front of each other
+    const SlotWord<T> sw(uniform(Pr.n));
     int key[S];
     int mine = 0;
 #pragma unroll
@@ -478,7 +480,7 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
 #pragma unroll
     for (int s = 0; s < S; ++s)
         if (key[s] != kEmpty) {
-            if (pos < P) row.cols[pos] = key[s];
+            if (pos < P) row.words[pos] = sw.pack(key[s], static_cast<int>(threadIdx.x) * S + s);
             ++pos;
         }
     __syncthreads();
@@ -487,13 +489,13 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     const int n = min(found, P);
     const int w = min(n, cn);
     const int mine0 = wave * B + lane * E;
-    int x[E];
+    uint32_t x[E];
 #pragma unroll
-    for (int s = 0; s < E; ++s) x[s] = mine0 + s < n ? row.cols[mine0 + s] : INT_MAX;
+    for (int s = 0; s < E; ++s) x[s] = mine0 + s < n ? row.words[mine0 + s] : ~0u;
     if (wave * B < n) {
         wave_sort<E>(x);
 #pragma unroll
-        for (int s = 0; s < E; ++s) row.cols[mine0 + s] = x[s];
+        for (int s = 0; s < E; ++s) row.words[mine0 + s] = x[s];
     }
     __syncthreads();
     if (wave * B < n) {
@@ -505,17 +507,17 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
             const int other = (wave + o) % kWaves;
             if (other * B >= n) continue;
             int at[E];
-            lower_bound_all<B, E>(row.cols + other * B, x, at);
+            lower_bound_all<B, E>(row.words + other * B, x, at);
 #pragma unroll
             for (int s = 0; s < E; ++s) {
                 // (a block of B columns may hold none as large: B steps of the search end one short)
-                at[s] += row.cols[other * B + at[s]] < x[s] ? 1 : 0;
+                at[s] += row.words[other * B + at[s]] < x[s] ? 1 : 0;
                 rank[s] += at[s];
             }
         }
 #pragma unroll
         for (int s = 0; s < E; ++s)
-            if (mine0 + s < n) row.slots[rank[s]] = static_cast<unsigned short>(table_find<T>(row.keys, x[s]));
+            if (mine0 + s < n) row.slots[rank[s]] = static_cast<unsigned short>(sw.slot(row.keys, x[s]));
     }
     __syncthreads();
     const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);

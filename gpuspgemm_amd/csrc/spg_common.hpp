@@ -349,14 +349,14 @@ __device__ __forceinline__ int wave_rank_add(int* cnt, int bin) {
 // Lower bounds of keys[J0, J0 + N), searched in lockstep: each halving step
 // reads the probes of all N keys at once, so a lane waits log2(P) LDS round
 // trips for the N keys instead of N * log2(P).
-template <int P, int N, int J0 = 0, int K>
-__device__ __forceinline__ void lower_bound_all(const int* cols, const int (&key)[K], int (&pos)[N]) {
+template <int P, int N, int J0 = 0, int K, typename X>
+__device__ __forceinline__ void lower_bound_all(const X* cols, const X (&key)[K], int (&pos)[N]) {
     static_assert(J0 + N <= K, "key range out of bounds");
 #pragma unroll
     for (int j = 0; j < N; ++j) pos[j] = 0;
 #pragma unroll
     for (int step = P >> 1; step > 0; step >>= 1) {
-        int probe[N];
+        X probe[N];
 #pragma unroll
         for (int j = 0; j < N; ++j) probe[j] = cols[pos[j] + step - 1];
 #pragma unroll

@@ -70,28 +70,29 @@ __device__ __forceinline__ uint32_t slot24(int key) {
 }
 
 // Slots of N keys in an LDS table of T slots (open addressing, linear
-// probing), inserting those that are new.  The probes of all keys advance
-// together, each a compare-and-swap; the lanes still probing are kept as
-// scalar masks, so that a key whose lanes are all done costs nothing more.
-// The table never fills (its row has fewer distinct columns than T).
-// With COUNT, `fresh` grows by the number of keys the wave inserted.
+// probing), inserting those that are new; ok[j]: the lanes that have a key j.
+// The probes of all keys advance together, each a compare-and-swap.  Lane
+// sets are scalar masks throughout (a ballot of one comparison is that
+// comparison's result register, so combining them costs no vector
+// instruction), and a key whose lanes are all done costs nothing more.
+// The table never fills (its row has fewer distinct columns than T).  With
+// COUNT, `fresh` grows by the number of keys the wave inserted.
 template <int T, int N, bool COUNT = false>
-__device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const bool (&ok)[N], uint32_t (&h)[N],
-                                            int& fresh) {
+__device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const unsigned long long (&ok)[N],
+                                            uint32_t (&h)[N], int& fresh) {
     int old[N];
-    unsigned long long pend[N];
+    unsigned long long pend[N], any = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         h[j] = slot24<T>(key[j]);
-        if (ok[j]) old[j] = atomicCAS(tab + h[j], kEmpty, key[j]);
+        if (in_mask(ok[j])) old[j] = atomicCAS(tab + h[j], kEmpty, key[j]);
     }
-    unsigned long long any = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        const bool on = ok[j] && old[j] != kEmpty && old[j] != key[j];
-        if constexpr (COUNT) fresh += __popcll(__ballot(ok[j] && old[j] == kEmpty));
-        h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
-        pend[j] = __ballot(on);
+        const unsigned long long taken = __ballot(old[j] != kEmpty);
+        if constexpr (COUNT) fresh += __popcll(ok[j] & ~taken);
+        pend[j] = ok[j] & taken & __ballot(old[j] != key[j]);
+        h[j] = (h[j] + (in_mask(pend[j]) ? 1u : 0u)) & (T - 1);
         any |= pend[j];
     }
     while (any) {
@@ -101,16 +102,34 @@ __device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const
         any = 0;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            if (!pend[j]) continue;
-            const bool was = in_mask(pend[j]);
-            const bool on = was && old[j] != kEmpty && old[j] != key[j];
-            if constexpr (COUNT) fresh += __popcll(__ballot(was && old[j] == kEmpty));
-            h[j] = (h[j] + (on ? 1u : 0u)) & (T - 1);
-            pend[j] = __ballot(on);
-            any |= pend[j];
+            if (pend[j]) {
+                const unsigned long long taken = __ballot(old[j] != kEmpty);
+                if constexpr (COUNT) fresh += __popcll(pend[j] & ~taken);
+                pend[j] &= taken & __ballot(old[j] != key[j]);
+                h[j] = (h[j] + (in_mask(pend[j]) ? 1u : 0u)) & (T - 1);
+                any |= pend[j];
+            }
         }
     }
 }
+
+// A column as the sort carries it: above its table slot where both fit one
+// word (B has fewer columns than leave room for the slot; all ones marks no
+// column), alone otherwise, and then its slot is looked up again after the
+// sort (four LDS probes a column in the worst lane of a wave).
+template <int T>
+struct SlotWord {
+    static constexpr int kBits = __builtin_ctz(T);
+    int shift;       // scalar: kBits or 0
+    uint32_t slots;  // scalar: T - 1 or 0
+    __device__ __forceinline__ explicit SlotWord(int columns)
+        : shift(columns < (1 << (32 - kBits)) ? kBits : 0), slots(shift ? T - 1 : 0) {}
+    __device__ __forceinline__ uint32_t pack(int key, int slot) const {
+        return static_cast<uint32_t>(key) << shift | (static_cast<uint32_t>(slot) & slots);
+    }
+    __device__ __forceinline__ int column(uint32_t w) const { return static_cast<int>(w >> shift); }
+    __device__ __forceinline__ uint32_t slot(const int* tab, uint32_t w) const;
+};
 
 // Slot of a key that is in the table.
 template <int T>
@@ -118,6 +137,10 @@ __device__ __forceinline__ uint32_t table_find(const int* tab, int key) {
     uint32_t h = slot24<T>(key);
     while (lds_load(tab + h) != key) h = (h + 1) & (T - 1);
     return h;
+}
+template <int T>
+__device__ __forceinline__ uint32_t SlotWord<T>::slot(const int* tab, uint32_t w) const {
+    return shift ? w & (T - 1) : table_find<T>(tab, static_cast<int>(w));
 }
 
 // Sort of 64 * E keys, lane l holding keys l*E .. l*E + E-1 of the result
@@ -273,7 +296,7 @@ struct alignas(16) WaveRow {
     int keys[T];
     union {
         WaveChunk<true> walk;
-        int cols[P];
+        uint32_t words[P];
     };
 };
 constexpr int wave_row_bytes(int p, int t) {
@@ -294,7 +317,7 @@ struct alignas(16) GroupRow {
     union {
         WaveChunk<true> walk[WAVES];
         struct {
-            int cols[P];
+            uint32_t words[P];
             unsigned short slots[P];
         };
     };
@@ -321,7 +344,7 @@ struct WaveOperands {
 };
 
 // The products of A's entries [a0, a1), in rounds of N * 64:
-// f(key[N], prod[N], ok[N]).  The wave takes 64 entries at a time, one to a
+// f(key[N], prod[N], ok[N]), ok[j] the lanes with a product j.  The wave takes 64 entries at a time, one to a
 // lane; entries with an empty row of B drop out.  A product's entry is the
 // number of entries that start at or before it (less one): the chunk's
 // starts are marked in a bitmap, 64 products to a word and one position
@@ -386,23 +409,23 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
                         __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(w),
                                                   static_cast<unsigned>(wc->before[r * N + j]))));
                 }
-                bool ok[N];
+                unsigned long long ok[N];
                 int key[N];
                 V bv[N];
 #pragma unroll
                 for (int j = 0; j < N; ++j) {
                     // a lane past the last product reads B's first entry
                     const int p0 = base + j * kWave;
-                    ok[j] = lane < in_win - p0;
+                    ok[j] = __ballot(lane < in_win - p0);
                     if constexpr (WIDE) {
                         const int pos = wc->ent[en[j]].d + lane + (win + p0);
-                        const int at = ok[j] ? pos : 0;
+                        const int at = in_mask(ok[j]) ? pos : 0;
                         key[j] = W.b_col[at];
                         if constexpr (VALS) bv[j] = W.b_val[at];
                     } else {
                         const uint32_t pos = static_cast<uint32_t>(wc->ent[en[j]].d) + static_cast<uint32_t>(lane * 4) +
                                              static_cast<uint32_t>((win + p0) * 4);
-                        const uint32_t o = ok[j] ? pos : 0u;
+                        const uint32_t o = in_mask(ok[j]) ? pos : 0u;
                         key[j] = *(const int32_t SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_col + o);
                         if constexpr (VALS)
                             bv[j] = *(const V SPG_GLOBAL*)((const char SPG_GLOBAL*)W.b_val +
