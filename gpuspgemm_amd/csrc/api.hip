@@ -808,7 +808,7 @@ struct Job : JobBase {
     std::vector<Prob<V>> probs;
     std::vector<Tile> tiles;
     ProbSet<V> ps{};
-    long long total_rows = 0;
+    long long total_rows = 0, total_entries = 0;  // of A
     int n_tiles = 0;
     bool batch = false;
     bool empty = false;
@@ -907,7 +907,7 @@ struct Job : JobBase {
         }
         L.meta_clean = false;
         prof.begin("nip", total_rows, n_tiles, s);
-        launch_nip<V>(ps, sym, meta, items1, static_cast<int>(total_rows), s);
+        launch_nip<V>(ps, sym, meta, items1, static_cast<int>(total_rows), total_entries, s);
         prof.end();
         const int n_multi = sym.n - 1;
         int grid = c.cus * c.occ_sym_multi;
@@ -946,7 +946,7 @@ struct Job : JobBase {
     // contents (operand descriptors, tiles) are copied from pinned host
     // memory by the phase itself and so are not part of it.
     std::vector<int64_t> signature(int phase) const {
-        std::vector<int64_t> k{phase, static_cast<int64_t>(sizeof(V)), count, n_tiles, total_rows,
+        std::vector<int64_t> k{phase, static_cast<int64_t>(sizeof(V)), count, n_tiles, total_rows, total_entries,
                                reinterpret_cast<int64_t>(L.scratch), reinterpret_cast<int64_t>(L.h_stage)};
         const BinTable& t = phase == 0 ? sym : num;
         k.push_back(t.n);
@@ -1045,6 +1045,7 @@ struct Job : JobBase {
         const size_t o_nip = take(sizeof(int32_t) * M);
         size_t nnz_a = 0;
         for (int i = 0; i < count; ++i) nnz_a += static_cast<size_t>(A[i].nnz);
+        total_entries = static_cast<long long>(nnz_a);
         const size_t o_bref = take(sizeof(long long) * nnz_a);
         const size_t o_it1 = take(sizeof(int2) * M * sym.n);  // a region of M items per symbolic bin
         const size_t o_it2 = take(sizeof(RowItem) * M);

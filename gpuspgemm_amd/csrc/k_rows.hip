@@ -22,9 +22,10 @@ __global__ __launch_bounds__(256) void k_clear(DevMeta* meta, int from_word) {
 // items[b * bin_cap, (b + 1) * bin_cap) with bin_cap >= the total row
 // count, so a tile's place in it is one atomic add on the bin's count and
 // no offsets have to be known beforehand.
+// A workgroup takes `parts` to the tile, tile / parts rows each.
 template <typename V>
 __global__ __launch_bounds__(kRowThreads) void k_nip(ProbSet<V> ps, BinTable sym, DevMeta* meta,
-                                                     int2* __restrict__ items, int bin_cap) {
+                                                     int2* __restrict__ items, int bin_cap, int parts) {
     __shared__ int s_cnt[kMaxBins];
     __shared__ int s_base[kMaxBins];
     __shared__ int s_max;
@@ -41,11 +42,16 @@ __global__ __launch_bounds__(kRowThreads) void k_nip(ProbSet<V> ps, BinTable sym
     }
     __syncthreads();
 
-    const Tile t = ps.tile(blockIdx.x);
+    Tile t = ps.tile(blockIdx.x / parts);
     const GProb<V> P = ps.get(t.inst);
-    // NIP of each lane's rows.  A wave takes 64 * kPer consecutive rows, kPer
-    // consecutive ones per lane, so the wave's entries are one consecutive
-    // range of A's columns.  The wave walks that range in rounds of kRound
+    const int part_rows = kTileRows / parts;
+    const int part0 = blockIdx.x % parts * part_rows;
+    t.row0 += part0;
+    t.rows = max(0, min(part_rows, t.rows - part0));
+    // NIP of each lane's rows.  A wave takes part_rows / waves consecutive
+    // rows, kPer consecutive ones per lane (the last lanes none when these are
+    // fewer than 64 * kPer), so the wave's entries are one consecutive range
+    // of A's columns.  The wave walks that range in rounds of kRound
     // entries side by side: coalesced loads of A's columns, a gather of B's
     // row pointers each (every load of the round in flight at once),
     // coalesced stores of the (start, length) of every entry's row of B (the
@@ -57,10 +63,12 @@ __global__ __launch_bounds__(kRowThreads) void k_nip(ProbSet<V> ps, BinTable sym
     constexpr int kPer = kTileRows / kRowThreads;
     long long* pref = s_pref[threadIdx.x / kWave];
     int* lens = reinterpret_cast<int*>(pref);  // the round's lengths, in its first half
-    const int wrow = (threadIdx.x / kWave) * (kWave * kPer) + lane_id() * kPer;  // the lane's first row in the tile
+    const int wave_rows = part_rows / (kRowThreads / kWave);
+    const int wrow0 = static_cast<int>(threadIdx.x / kWave) * wave_rows;
+    const int wrow = wrow0 + min(lane_id() * kPer, wave_rows);  // the lane's first row in the part
     int bound[kPer + 1];  // entry bounds of the lane's rows
 #pragma unroll
-    for (int j = 0; j <= kPer; ++j) bound[j] = P.a_rpt[t.row0 + min(wrow + j, t.rows)];
+    for (int j = 0; j <= kPer; ++j) bound[j] = P.a_rpt[t.row0 + min(min(wrow + j, wrow0 + wave_rows), t.rows)];
     long long s[kPer] = {};
     const int g0 = __shfl(bound[0], 0), g1 = __shfl(bound[kPer], kWave - 1);
     for (int rb = g0; rb < g1; rb += kRound) {
@@ -125,7 +133,7 @@ __global__ __launch_bounds__(kRowThreads) void k_nip(ProbSet<V> ps, BinTable sym
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
         const int r = wrow + j;
-        const bool valid = r < t.rows;
+        const bool valid = r < min(wrow0 + wave_rows, t.rows);
         const int row = t.row0 + r;
         bin[j] = -1;
         if (valid) {
@@ -467,9 +475,25 @@ void launch_clear(DevMeta* meta, int from_word, hipStream_t s) {
     hipLaunchKernelGGL(k_clear, dim3(1), dim3(256), 0, s, meta, from_word);
 }
 
+// Parts per tile: a wave's rows are walked in rounds of 512 entries, one
+// after the other, so a tile of dense rows is split until a wave has at most
+// two rounds, unless the workgroups then pass kNipMaxGroups: each adds to the
+// same few counters, about 10 ns apiece, which they hide up to there.
+// (32^3 stencil, 16 tiles: 32.5 -> 16.5 us; 27^3 x 3 unknowns, 29 tiles of 81
+// entries a row: 72 -> 21 us; 96^3 stencil, 432 tiles: 104 -> 91 us.)
+constexpr int kNipMaxGroups = 2048;
+constexpr long long kNipWaveEntries = 1024;
 template <typename V>
-void launch_nip(const ProbSet<V>& ps, const BinTable& sym, DevMeta* meta, int2* items, int bin_cap, hipStream_t s) {
-    hipLaunchKernelGGL(k_nip<V>, dim3(ps.n_tiles), dim3(kRowThreads), 0, s, ps, sym, meta, items, bin_cap);
+void launch_nip(const ProbSet<V>& ps, const BinTable& sym, DevMeta* meta, int2* items, int bin_cap, long long entries,
+                hipStream_t s) {
+    constexpr int kWaves = kRowThreads / kWave;
+    constexpr int kMaxParts = kTileRows / (kWaves * 16);  // at least 16 rows to a wave
+    int parts = 1;
+    while (parts < kMaxParts && 2 * parts * ps.n_tiles <= kNipMaxGroups &&
+           entries > kNipWaveEntries * kWaves * parts * ps.n_tiles)
+        parts *= 2;
+    hipLaunchKernelGGL(k_nip<V>, dim3(ps.n_tiles * parts), dim3(kRowThreads), 0, s, ps, sym, meta, items, bin_cap,
+                       parts);
 }
 
 
@@ -491,7 +515,8 @@ void launch_scan_apply(const ProbSet<V>& ps, const BinTable& num, DevMeta* meta,
 }
 
 #define SPG_INSTANTIATE_ROWS(V)                                                                        \
-    template void launch_nip<V>(const ProbSet<V>&, const BinTable&, DevMeta*, int2*, int, hipStream_t); \
+    template void launch_nip<V>(const ProbSet<V>&, const BinTable&, DevMeta*, int2*, int, long long,    \
+                                hipStream_t);                                                          \
     template void launch_scan_count<V>(const ProbSet<V>&, const BinTable&, DevMeta*, long long*, int,  \
                                        hipStream_t);                                                   \
     template void launch_scan_apply<V>(const ProbSet<V>&, const BinTable&, DevMeta*, long long*,       \

@@ -182,9 +182,10 @@ void launch_total_nip(const int32_t* a_rpt, const int32_t* a_col, const int32_t*
                       unsigned long long* out, hipStream_t s);
 
 // NIP per row and the scatter into the symbolic bin lists (bin b's list
-// starts at items + b * bin_cap)
+// starts at items + b * bin_cap); entries: of A, over all products
 template <typename V>
-void launch_nip(const ProbSet<V>& ps, const BinTable& sym, DevMeta* meta, int2* items, int bin_cap, hipStream_t s);
+void launch_nip(const ProbSet<V>& ps, const BinTable& sym, DevMeta* meta, int2* items, int bin_cap, long long entries,
+                hipStream_t s);
 template <typename V>
 void launch_scan_count(const ProbSet<V>& ps, const BinTable& num, DevMeta* meta, long long* tile_sums,
                        int after_fail, hipStream_t s);

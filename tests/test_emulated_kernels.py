@@ -245,6 +245,23 @@ def test_nip_per_row(emu, tmp_path):
     assert [int(x) for x in got.split()] == want, line
 
 
+def test_nip_of_dense_tiles(emu, tmp_path):
+    """Tiles of dense rows are split over several workgroups of the NIP pass
+    (here 2,100 rows of 0 to 90 entries: 47 entries a row, four parts a
+    tile); the last tile ends inside its first part."""
+    rng = np.random.default_rng(43)
+    n = 300
+    B = gen.random_csr(n, 50, 0.02, seed=44, empty_rows=0.2)
+    a_len = rng.integers(0, 91, 2100)
+    rpt = np.concatenate([[0], np.cumsum(a_len)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in a_len]).astype(np.int32)
+    A = HostCSR(2100, n, rpt, col, rng.uniform(-1, 1, col.size))
+    nip = oracle.nip_rows(A, B)
+    out = run_emu(emu, tmp_path, A, B, env={"SPG_LOG_LEVEL": "debug"})
+    line = next(x for x in out.splitlines() if "symbolic phase" in x)
+    assert f"NIP {int(nip.sum())} (max {int(nip.max())} per row)" in line, line
+
+
 def test_scanned_tile_prefix(emu, tmp_path):
     """The scan stage reads each tile's prefix off one scanned array of tile
     sums, the path of multiplies of 2048 tiles or more, forced here from one
