@@ -530,6 +530,100 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     __syncthreads();  // LDS is reused by the next row
 }
 
+// Rows of up to P columns whose table takes most of LDS (a workgroup of 16
+// waves on a CU of its own): the columns are found in LDS and compacted
+// through C.col, their sorted list takes the table's place, and a second walk
+// finds every product in it (15 LDS steps, four products of a lane in
+// lockstep) and adds it to C.val in memory.  The searches are what the
+// global-memory path below is slow at: a row of 16,767 products and 14,389
+// columns took 460 us there, most of it dependent reads of the sorted list.
+template <typename V, int WG, int P, int T, int N>
+__device__ __forceinline__ void symnum_long_row(const ProbSet<V>& ps, const RowItem* __restrict__ items, int idx,
+                                                LongRow<T, WG / kWave>& row, int* s_tmp, DevMeta* meta) {
+    constexpr int kWaves = WG / kWave;
+    static_assert(P < T && T % (4 * WG) == 0, "the table keeps free slots");
+    const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+    typedef int Words __attribute__((vector_size(16)));
+    for (int i = threadIdx.x; i < T / 4; i += WG)
+        reinterpret_cast<Words*>(row.keys)[i] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+    const RowItem it = load_item(items, idx);
+    const GProb<V> Pr = ps.get(uniform(it.inst));
+    const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+    const int a0 = uniform(it.a0), a1 = uniform(it.a1), cn = uniform(it.cn);
+    const bool by_chunk = wave_by_chunk<kWaves>(a1 - a0, uniform(it.nip));
+    const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);
+    const auto cval = uniform_ptr(Pr.c_val) + uniform(it.c0);
+    for (int j = threadIdx.x; j < cn; j += WG) cval[j] = V(0);
+    __syncthreads();
+    // (the walk without values uses the front of the same metadata)
+    wave_products<V, N, false>(
+        W, a0, a1, reinterpret_cast<WaveChunk<false>*>(&row.walk[wave]),
+        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) {
+            uint32_t h[N];
+            int fresh = 0;
+            table_slots<T>(row.keys, key, ok, h, fresh);
+        },
+        wave, kWaves, by_chunk);
+    __syncthreads();
+    // the occupied slots into C.col, unsorted, WG * 4 slots at a time
+    int found = 0;
+    for (int base = 0; base < T; base += 4 * WG) {
+        const Words k = reinterpret_cast<const Words*>(row.keys)[base / 4 + threadIdx.x];
+        int mine = 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) mine += k[s] != kEmpty ? 1 : 0;
+        int total;
+        int pos = found + group_excl_scan<WG>(mine, threadIdx.x, s_tmp, total);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (k[s] != kEmpty) {
+                if (pos < cn) ccol[pos] = k[s];
+                ++pos;
+            }
+        found += total;
+    }
+    if (threadIdx.x == 0 && found != cn) atomicOr(&meta->flags.v, kFlagMismatch);
+    const int n = min(found, cn);
+    __threadfence();  // C.val is zero, C.col written, before other waves read or add
+    __syncthreads();
+    // the smallest power of two of columns that holds them all
+    auto sort_as = [&](auto size) {
+        constexpr int kP = decltype(size)::value;
+        for (int j = threadIdx.x; j < kP; j += WG)
+            row.keys[j] = j < n ? __hip_atomic_load(ccol + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : INT_MAX;
+        __syncthreads();
+        bitonic_sort_block<kP, WG>(row.keys, threadIdx.x);
+    };
+    if (n <= T / 2)
+        sort_as(std::integral_constant<int, T / 2>{});
+    else
+        sort_as(std::integral_constant<int, T>{});
+    for (int j = threadIdx.x; j < n; j += WG) ccol[j] = row.keys[j];
+    const int half = n <= T / 2 ? T / 4 : T / 2;
+    wave_products<V, N, true>(
+        W, a0, a1, &row.walk[wave],
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
+            int pos[N];
+#pragma unroll
+            for (int j = 0; j < N; ++j) pos[j] = 0;
+            for (int step = half; step > 0; step >>= 1) {
+                int probe[N];
+#pragma unroll
+                for (int j = 0; j < N; ++j) probe[j] = row.keys[pos[j] + step - 1];
+#pragma unroll
+                for (int j = 0; j < N; ++j) pos[j] += probe[j] < key[j] ? step : 0;
+            }
+#pragma unroll
+            for (int j = 0; j < N; ++j)
+                if (in_mask(ok[j]) && pos[j] < n)
+                    __hip_atomic_fetch_add(cval + pos[j], static_cast<V>(prod[j]), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+        },
+        wave, kWaves, by_chunk);
+    __syncthreads();  // LDS is reused by the next row
+}
+
 // The rows [first, end) of one unit of variant VV.
 template <typename V, int VV>
 __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem* __restrict__ items, int first,
@@ -540,6 +634,9 @@ __device__ __forceinline__ void symnum_unit(const ProbSet<V>& ps, const RowItem*
         if (first + wave < end)
             symnum_wave_row<V, kV.p, kV.t, kV.pmax>(ps, items, first + wave,
                                                     reinterpret_cast<WaveRow<kV.p, kV.t>*>(smem)[wave], meta);
+    } else if constexpr (num_is_long(kV)) {
+        symnum_long_row<V, kV.wg, kV.p, kV.t, kV.pmax>(ps, items, first,
+                                                       *reinterpret_cast<LongRow<kV.t, kV.wg / kWave>*>(smem), s_tmp, meta);
     } else if constexpr (num_is_group(kV)) {
         symnum_group_row<V, kV.wg, kV.p, kV.t, kV.pmax>(
             ps, items, first, *reinterpret_cast<GroupRow<kV.p, kV.t, kV.wg / kWave>*>(smem), meta);
@@ -565,7 +662,7 @@ __global__ __launch_bounds__(kNumVariants[VV].wg) SPG_WAVES_PER_EU(kNumMinWaves[
 }
 
 #define SPG_NUM_VARIANTS(X) \
-    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19)
+    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20)
 
 // Several bins of the fused pass in one launch, a workgroup per unit.
 // Each XCD gets a contiguous slice of every bin (balanced work across the

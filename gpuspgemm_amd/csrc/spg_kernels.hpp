@@ -23,7 +23,9 @@ struct NumVariant {
 // Rows of one wave each (wg / r == 64): see symnum_wave_row; rows that a
 // workgroup's waves share, with values in the table: symnum_group_row.
 constexpr bool num_is_wave(const NumVariant& v) { return v.wg / v.r == kWave; }
-constexpr bool num_is_group(const NumVariant& v) { return v.wg / v.r > kWave && v.t > 0; }
+constexpr bool num_is_group(const NumVariant& v) { return v.wg / v.r > kWave && v.t > 0 && v.t <= 4096; }
+// The longest rows that fit LDS: only the columns do, see symnum_long_row.
+constexpr bool num_is_long(const NumVariant& v) { return v.t > 4096; }
 
 
 // Symbolic (count) variants.  0..8 run inside one launch of 256-thread
@@ -58,7 +60,7 @@ constexpr bool sym_is_group(const SymVariant& v) { return v.wg / v.r > kWave; }
 
 // Fused sorted-columns + numeric variants, one kernel each: all use 256
 // threads except 9 (a 1024-thread workgroup per row); rows above every
-// capacity use global-memory tables (variant 20).  A row whose products fit
+// capacity use global-memory tables (variant 21).  A row whose products fit
 // in one chunk and in lanes * pmax keeps them in registers between the two
 // halves.  Variants 10..18 cover the small capacities with 2 to 32 lanes
 // per row; the tuner picks among them per bin.
@@ -68,8 +70,9 @@ constexpr NumVariant kNumVariants[] = {
     {256, 1, 2048, 256, 8}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
     {256, 8, 32, 32, 4},    {256, 4, 64, 64, 4, 128}, {256, 64, 8, 8, 4},    {256, 128, 8, 4, 8},
     {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},  {256, 1, 512, 64, 4, 1024},
+    {1024, 1, 26214, 64, 4, 32768},
 };
-constexpr int kNumLdsVariants = 20;  // variants with an LDS kernel (0..19)
+constexpr int kNumLdsVariants = 21;  // variants with an LDS kernel (0..20)
 // Waves per SIMD that each fused variant's kernel must keep (its register
 // budget is 512 / waves VGPRs).  Fetching a lane's products as one batch
 // of loads (every load in flight before the first multiply) needs more
@@ -77,8 +80,8 @@ constexpr int kNumLdsVariants = 20;  // variants with an LDS kernel (0..19)
 // the variant had with the one-by-one fetch, and the compiler schedules
 // the batch within it.  Measured on gfx950: the 96^3 stencil's fused pass
 // 3.23 -> 2.81 ms, the power-law's 198k-row bin 70 -> 53 us.
-constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 5, 3, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 8};
-constexpr int kNumGlobalVariant = 20;
+constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 5, 3, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 8, 4};
+constexpr int kNumGlobalVariant = 21;
 
 // Fused variants whose bins share one launch.  Set 0, small rows (256
 // threads, up to 32 lanes per row, about 64 VGPRs): their bins hold most
@@ -129,7 +132,8 @@ constexpr int padded_row_ints(int bytes) {
 // Fused variant: table 2p ints (reused for p sums in double), sorted
 // list p ints, chunk metadata when the row has more than one lane.
 constexpr int num_row_ints(const NumVariant& v) {
-    return num_is_group(v) ? group_row_bytes(v.p, v.t, v.wg / kWave) / 4
+    return num_is_long(v) ? long_row_bytes(v.t, v.wg / kWave) / 4
+         : num_is_group(v) ? group_row_bytes(v.p, v.t, v.wg / kWave) / 4
          : num_is_wave(v) ? wave_row_bytes(v.p, v.t) / 4
                            : padded_row_ints(12 * v.p + (v.wg / v.r > 1 ? 16 * v.ec : 0));
 }

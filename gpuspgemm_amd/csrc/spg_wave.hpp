@@ -333,6 +333,20 @@ static_assert(sizeof(GroupRow<512, 1024, 4>) == group_row_bytes(512, 1024, 4) &&
                   sizeof(GroupRow<1024, 2048, 4>) == group_row_bytes(1024, 2048, 4),
               "LDS size of a workgroup's row");
 
+// A row whose columns fill most of LDS: the table, then the sorted columns in
+// its place.
+template <int T, int WAVES>
+struct alignas(16) LongRow {
+    int keys[T];
+    WaveChunk<true> walk[WAVES];
+    int wave_sum[WAVES];
+};
+constexpr int long_row_bytes(int t, int waves) {
+    const int all = 4 * t + waves * (static_cast<int>(sizeof(WaveChunk<true>)) + 4);
+    return (all + 15) / 16 * 16;
+}
+static_assert(sizeof(LongRow<32768, 16>) == long_row_bytes(32768, 16), "LDS size of a long row");
+
 // Where a wave's walk reads (all scalar).
 template <typename V>
 struct WaveOperands {

@@ -247,15 +247,15 @@ def test_nip_per_row(emu, tmp_path):
 
 def test_nip_of_dense_tiles(emu, tmp_path):
     """Tiles of dense rows are split over several workgroups of the NIP pass
-    (here 2,100 rows of 0 to 90 entries: 47 entries a row, four parts a
-    tile); the last tile ends inside its first part."""
+    (here 1,100 rows of 0 to 90 entries, four parts of 512 rows): full
+    parts, one that the rows end in and an empty one."""
     rng = np.random.default_rng(43)
     n = 300
-    B = gen.random_csr(n, 50, 0.02, seed=44, empty_rows=0.2)
-    a_len = rng.integers(0, 91, 2100)
+    B = gen.random_csr(n, 50, 0.006, seed=44)
+    a_len = rng.integers(0, 91, 1100)
     rpt = np.concatenate([[0], np.cumsum(a_len)]).astype(np.int32)
     col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in a_len]).astype(np.int32)
-    A = HostCSR(2100, n, rpt, col, rng.uniform(-1, 1, col.size))
+    A = HostCSR(1100, n, rpt, col, rng.uniform(-1, 1, col.size))
     nip = oracle.nip_rows(A, B)
     out = run_emu(emu, tmp_path, A, B, env={"SPG_LOG_LEVEL": "debug"})
     line = next(x for x in out.splitlines() if "symbolic phase" in x)
