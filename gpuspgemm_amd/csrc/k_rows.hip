@@ -45,9 +45,9 @@ __global__ __launch_bounds__(kRowThreads) void k_nip(ProbSet<V> ps, BinTable sym
     Tile t = ps.tile(blockIdx.x / parts);
     const GProb<V> P = ps.get(t.inst);
     const int part_rows = kTileRows / parts;
-    const int part0 = blockIdx.x % parts * part_rows;
+    const int part0 = min(static_cast<int>(blockIdx.x) % parts * part_rows, t.rows);  // (a part past the tile is empty)
     t.row0 += part0;
-    t.rows = max(0, min(part_rows, t.rows - part0));
+    t.rows = min(part_rows, t.rows - part0);
     // NIP of each lane's rows.  A wave takes part_rows / waves consecutive
     // rows, kPer consecutive ones per lane (the last lanes none when these are
     // fewer than 64 * kPer), so the wave's entries are one consecutive range

@@ -101,6 +101,37 @@ static int noalloc(const std::string& fa, const std::string& fb, int repeat) {
     return bad;
 }
 
+// A batch of the given product behind one whose operands have no entries
+// (null column and value arrays).
+template <typename T>
+static int batch_after_empty(const std::string& fa, const std::string& fb) {
+    const auto ha = utils::HostCSR<T>::load_from_filename(fa);
+    const auto hb = utils::HostCSR<T>::load_from_filename(fb);
+    const auto da = ha.template to<utils::Location::Device>();
+    const auto db = hb.template to<utils::Location::Device>();
+    const auto ref = host::gustavson(ha, hb);
+    const auto absref = host::abs_product(ha, hb);
+    void* zero = nullptr;
+    const std::vector<int32_t> zeros(6, 0);
+    utils::handle_spg_error(spg_malloc(&zero, sizeof(int32_t) * 6), "malloc");
+    utils::handle_spg_error(spg_memcpy(zero, zeros.data(), sizeof(int32_t) * 6), "memcpy");
+    const spg_csr empty{0, 5, 5, static_cast<int32_t*>(zero), nullptr, nullptr};
+    const spg_csr As[2] = {empty, da.raw()}, Bs[2] = {empty, db.raw()};
+    spg_csr Cs[2] = {};
+    utils::handle_spg_error(spg_multiply_batched(2, As, Bs, Cs, sizeof(T) == 8 ? SPG_F64 : SPG_F32), "batched");
+    utils::HostCSR<T> hc(Cs[1].nnz, Cs[1].m, Cs[1].n);
+    utils::handle_spg_error(spg_memcpy(hc.rpt, Cs[1].rpt, sizeof(int32_t) * (hc.m + 1)), "memcpy");
+    utils::handle_spg_error(spg_memcpy(hc.col, Cs[1].col, sizeof(int32_t) * hc.nnz), "memcpy");
+    utils::handle_spg_error(spg_memcpy(hc.val, Cs[1].val, sizeof(T) * hc.nnz), "memcpy");
+    const auto e = host::errors(hc, ref, absref);
+    std::printf("batch: nnz %d and %d structure %s scaled_err %.3e\n", Cs[0].nnz, hc.nnz,
+                e.structure ? "identical" : "DIFFERENT", e.scaled);
+    utils::handle_spg_error(spg_csr_free(&Cs[0]), "free");
+    utils::handle_spg_error(spg_csr_free(&Cs[1]), "free");
+    utils::handle_spg_error(spg_free(zero), "free");
+    return e.structure && Cs[0].nnz == 0 && e.scaled <= (sizeof(T) == 8 ? 1e-12 : 1e-5) ? 0 : 1;
+}
+
 template <typename T>
 static int serve(const std::string& fa, const std::string& fb, int n, long long budget, int max_batch) {
     const auto ha = utils::HostCSR<T>::load_from_filename(fa);
@@ -175,7 +206,7 @@ int main(int argc, char** argv) {
         std::fprintf(stderr, "usage: %s A.csr B.csr [--f32] [--sym-table F] [--num-table F] [--repeat N]\n", argv[0]);
         return 2;
     }
-    bool f32 = false, graphs = false, use_noalloc = false;
+    bool f32 = false, graphs = false, use_noalloc = false, after_empty = false;
     int repeat = 1, serve_n = 0, max_batch = 1;
     long long budget = 0;
     for (int i = 3; i < argc; ++i) {
@@ -187,6 +218,8 @@ int main(int argc, char** argv) {
             utils::handle_spg_error(spg_set_tuning(a == "--sym-table" ? 0 : 1, t.c_str()), "set_tuning");
         } else if (a == "--graphs") {
             graphs = true;
+        } else if (a == "--batch-after-empty") {
+            after_empty = true;
         } else if (a == "--noalloc") {
             use_noalloc = true;
         } else if (a == "--repeat" && i + 1 < argc) {
@@ -205,6 +238,8 @@ int main(int argc, char** argv) {
         if (serve_n > 0)
             return f32 ? serve<float>(argv[1], argv[2], serve_n, budget, max_batch)
                        : serve<double>(argv[1], argv[2], serve_n, budget, max_batch);
+        if (after_empty)
+            return f32 ? batch_after_empty<float>(argv[1], argv[2]) : batch_after_empty<double>(argv[1], argv[2]);
         if (use_noalloc)
             return f32 ? noalloc<float>(argv[1], argv[2], repeat) : noalloc<double>(argv[1], argv[2], repeat);
         return f32 ? run<float>(argv[1], argv[2], repeat, graphs) : run<double>(argv[1], argv[2], repeat, graphs);

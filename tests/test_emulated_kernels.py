@@ -247,15 +247,18 @@ def test_nip_per_row(emu, tmp_path):
 
 def test_nip_of_dense_tiles(emu, tmp_path):
     """Tiles of dense rows are split over several workgroups of the NIP pass
-    (here 1,100 rows of 0 to 90 entries, four parts of 512 rows): full
-    parts, one that the rows end in and an empty one."""
+    (here 1,535 rows of 0 to 90 entries, eight parts of 256 rows): full
+    parts, one that the rows end in and two empty ones.  The first empty part
+    would start one past A's last row pointer, where AddressSanitizer sees a
+    read that is not clamped to the tile's end."""
     rng = np.random.default_rng(43)
     n = 300
     B = gen.random_csr(n, 50, 0.006, seed=44)
-    a_len = rng.integers(0, 91, 1100)
+    a_len = rng.integers(0, 91, 1535)
     rpt = np.concatenate([[0], np.cumsum(a_len)]).astype(np.int32)
     col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in a_len]).astype(np.int32)
-    A = HostCSR(1100, n, rpt, col, rng.uniform(-1, 1, col.size))
+    A = HostCSR(1535, n, rpt, col, rng.uniform(-1, 1, col.size))
+    assert col.size > 1024 * 16 * 4
     nip = oracle.nip_rows(A, B)
     out = run_emu(emu, tmp_path, A, B, env={"SPG_LOG_LEVEL": "debug"})
     line = next(x for x in out.splitlines() if "symbolic phase" in x)
@@ -391,6 +394,18 @@ def test_sorted_rows(emu, tmp_path, variant, products, columns):
     A, B = matrix(a_rows, 64, 95), matrix(b_rows, columns, 96)
     table = {1: f"{variant} {INT_MAX} {NUM[variant][2]}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
     run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A, B, "--f32", tables=table))
+
+
+def test_batch_behind_a_product_without_entries(emu, tmp_path):
+    """A batch whose first product has no entries (null arrays): a wave of a
+    fused unit that has no row sees item zero, instance zero, and must not
+    read that product's B.  Five rows fill the first wave of a unit in part
+    and leave the others without one; 20 and 40 products a row too."""
+    for i, k in enumerate((2, 4, 6)):
+        A = gen.uniform8(m=5, per_row=k, seed=3, n=64)
+        B = gen.uniform8(m=64, per_row=k, seed=4, n=640)
+        (tmp_path / str(i)).mkdir()
+        run_emu(emu, tmp_path / str(i), A, B, "--batch-after-empty")
 
 
 def test_symbolic_overflow_moves_to_the_largest_table(emu, tmp_path):
