@@ -237,6 +237,7 @@ __device__ __forceinline__ void symnum_rows(const ProbSet<V>& ps, const RowItem*
     const bool active = idx < end;
     const RowItem it = active ? load_item(items, idx) : RowItem{0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (L >= 8 && L < kWave && P == L) {
+        if (__ballot(active) == 0) return;  // no row, and so no product whose B could be read
         const GProb<V> Pu = ps.get(uniform(it.inst));
         if (sorted_fits<V, L, 1>(Pu, it, active)) {
             static_assert(kWave / L * ROW_INTS * 4 >= static_cast<int>(sizeof(SortSlots<1>)) &&
