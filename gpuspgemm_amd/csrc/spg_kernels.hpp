@@ -67,9 +67,9 @@ constexpr bool sym_is_group(const SymVariant& v) { return v.wg / v.r > kWave; }
 constexpr NumVariant kNumVariants[] = {
     {256, 256, 8, 4, 16},   {256, 128, 16, 4, 16}, {256, 64, 32, 8, 16},  {256, 32, 64, 16, 16},
     {256, 16, 128, 32, 16}, {256, 4, 128, 64, 4, 256}, {256, 4, 256, 64, 4, 512}, {256, 1, 1024, 64, 4, 2048},
-    {256, 1, 2048, 256, 8}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
+    {256, 1, 512, 64, 4, 1024}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
     {256, 8, 32, 32, 4},    {256, 4, 64, 64, 4, 128}, {256, 64, 8, 8, 4},    {256, 128, 8, 4, 8},
-    {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},  {256, 1, 512, 64, 4, 1024},
+    {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},  {256, 1, 2048, 256, 8},
     {1024, 1, 26214, 64, 4, 32768},
 };
 constexpr int kNumLdsVariants = 21;  // variants with an LDS kernel (0..20)
@@ -80,7 +80,7 @@ constexpr int kNumLdsVariants = 21;  // variants with an LDS kernel (0..20)
 // the variant had with the one-by-one fetch, and the compiler schedules
 // the batch within it.  Measured on gfx950: the 96^3 stencil's fused pass
 // 3.23 -> 2.81 ms, the power-law's 198k-row bin 70 -> 53 us.
-constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 5, 3, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 8, 4};
+constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 5, 8, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 3, 4};
 constexpr int kNumGlobalVariant = 21;
 
 // Fused variants whose bins share one launch.  Set 0, small rows (256
