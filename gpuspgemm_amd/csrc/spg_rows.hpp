@@ -1,6 +1,8 @@
-// Row-level building blocks shared by the symbolic and fused passes.
+// Row-level building blocks of the rows that part of a wave, or a workgroup
+// in step, works on (rows of one wave and of waves that share a row walk on
+// their own: spg_wave.hpp).
 //
-// A row of C is worked on by a group of L consecutive lanes (L <= 64: the
+// A row of C is worked on by a group of L consecutive lanes (L < 64: the
 // group lives inside one wave and synchronises at wave level; L > 64: the
 // group is the whole workgroup).  Its products a_ik * b_kj are enumerated
 // flat: the group loads the metadata of EC entries of A's row at once (B
@@ -8,14 +10,8 @@
 // lengths, and lane lr handles products p = lr, lr + L, ...  Consecutive
 // lanes read consecutive entries of a B row (coalesced), every lane has up
 // to PMAX independent loads in flight, and short B rows leave no lane idle.
-// Product p belongs to the last entry that starts at or before p.  A group
-// of one whole wave (64 lanes) finds it by counting: per round of 64 * PMAX
-// products it sets one bit per entry start in an LDS bitmap, one 64-bit
-// word per slot, and the entry of p is the number of set bits up to p
-// (entries with empty B rows are dropped from the chunk first).  Narrower
-// and wider groups binary-search the entries' product offsets (measured:
-// for narrow groups, whose chunks are short, the counting costs more
-// registers than the search saves).
+// Product p belongs to the last entry that starts at or before p, found by
+// binary search over the entries' product offsets.
 #pragma once
 
 #include "spg_common.hpp"
@@ -77,24 +73,16 @@ __device__ __forceinline__ int group_excl_scan(int v, int lr, int* s_tmp, int& t
 // comes from P.bref[e] (start, length), recorded by the NIP pass.
 template <typename V, int EC, bool VALS>
 struct alignas(8) ChunkMeta {
-    // L != 64: exclusive prefix of B-row lengths, entries past the chunk
-    // holding the chunk total.  L == 64: the bitmap of entry starts of the
-    // current round (one 64-bit word per slot).
-    int off[EC];
-    // position in B of the entry's first product; L == 64: minus the
-    // entry's product offset
-    int d[EC];
+    int off[EC];  // exclusive prefix of B-row lengths, entries past the chunk holding the chunk total
+    int d[EC];    // position in B of the entry's first product
     V av[VALS ? EC : 1];     // a_ik
 };
 
 // Load entries [ebase, min(ebase + EC, a1)) of A's row into `cm`; returns
-// the chunk's product count.  Each lane loads EC/L consecutive entries.  A
-// group of one whole wave keeps only entries with a non-empty B row, in
-// order, and each lane gets the product offsets where its own entries
-// start (start[t], -1 for an empty one).
+// the chunk's product count.  Each lane loads EC/L consecutive entries.
 template <typename V, int L, int EC, bool VALS>
 __device__ __forceinline__ int load_chunk(const GProb<V>& P, int ebase, int a1, int lr,
-                                          ChunkMeta<V, EC, VALS>* cm, int* s_tmp, int (&start)[EC / L]) {
+                                          ChunkMeta<V, EC, VALS>* cm, int* s_tmp) {
     static_assert(EC % L == 0, "chunk must be a multiple of the group");
     constexpr int PER = EC / L;
     int len[PER], bs[PER];
@@ -111,7 +99,7 @@ __device__ __forceinline__ int load_chunk(const GProb<V>& P, int ebase, int a1, 
             if constexpr (VALS) a[t] = P.a_val[e];
         }
     }
-    int local = 0, filled = 0;
+    int local = 0;
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
         const bool in = ebase + lr * PER + t < a1;
@@ -120,34 +108,16 @@ __device__ __forceinline__ int load_chunk(const GProb<V>& P, int ebase, int a1, 
         av[t] = V(0);
         if constexpr (VALS) av[t] = in ? a[t] : V(0);
         local += len[t];
-        filled += len[t] > 0 ? 1 : 0;
     }
     int total;
     int run = group_excl_scan<L>(local, lr, s_tmp, total);
-    if constexpr (L == kWave) {
-        int n_filled;
-        int k = group_excl_scan<L>(filled, lr, s_tmp, n_filled);
 #pragma unroll
-        for (int t = 0; t < PER; ++t) {
-            start[t] = -1;
-            if (len[t] > 0) {
-                cm->d[k] = bs[t] - run;
-                if constexpr (VALS) cm->av[k] = av[t];
-                start[t] = run;
-                ++k;
-            }
-            run += len[t];
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < PER; ++t) {
-            const int e = lr * PER + t;
-            cm->off[e] = run;
-            cm->d[e] = bs[t];
-            if constexpr (VALS) cm->av[e] = av[t];
-            start[t] = run;
-            run += len[t];
-        }
+    for (int t = 0; t < PER; ++t) {
+        const int e = lr * PER + t;
+        cm->off[e] = run;
+        cm->d[e] = bs[t];
+        if constexpr (VALS) cm->av[e] = av[t];
+        run += len[t];
     }
     gsync<L>();
     return total;
@@ -171,60 +141,23 @@ __device__ __forceinline__ void chunk_find_all(const int* off, const int (&p)[PM
 }
 
 // Fetch up to PMAX products of a chunk: slot j holds product
-// base + j*L + lr.  ok[j] tells which slots are real.  `prior` counts the
-// entries that start before `base` (0 for a chunk's first round) and is
-// advanced past this round.  Three phases, so that a lane's gathers are in
-// flight together: the entry of every slot, then the loads of B's columns
-// and values for all slots, then the products a_ik * b_kj (a multiply next
-// to its load would wait for that load before the next one is issued).
+// base + j*L + lr.  ok[j] tells which slots are real.  Three phases, so that
+// a lane's gathers are in flight together: the entry of every slot, then the
+// loads of B's columns and values for all slots, then the products
+// a_ik * b_kj (a multiply next to its load would wait for that load before
+// the next one is issued).
 template <typename V, int L, int EC, int PMAX, bool VALS>
 __device__ __forceinline__ void fetch_products(const GProb<V>& P, ChunkMeta<V, EC, VALS>* cm, int total, int base,
-                                               int lr, const int (&start)[EC / L], int& prior, int (&key)[PMAX],
-                                               V (&prod)[PMAX], bool (&ok)[PMAX]) {
-    int e[PMAX];
-    if constexpr (L == kWave) {
-        // slot j covers bitmap word j; lane lr counts the set bits at or
-        // below its own position.  (Moving the word to scalar registers and
-        // counting with mbcnt measured slower.)
-        static_assert(kWave == 64, "one bitmap word per slot");
-        static_assert(2 * PMAX <= EC, "the bitmap lives in the chunk's offset array");
-        unsigned long long* bits = reinterpret_cast<unsigned long long*>(cm->off);
-        if (lr < PMAX) bits[lr] = 0;
-        wave_sync();
+                                               int lr, int (&key)[PMAX], V (&prod)[PMAX], bool (&ok)[PMAX]) {
+    int p[PMAX], e[PMAX];
 #pragma unroll
-        for (int t = 0; t < EC / L; ++t) {
-            const int q = start[t] - base;
-            if (start[t] >= 0 && q >= 0 && q < L * PMAX) atomicOr(&bits[q >> 6], 1ull << (q & 63));
-        }
-        wave_sync();
-        unsigned long long w[PMAX];
-#pragma unroll
-        for (int j = 0; j < PMAX; ++j) w[j] = bits[j];
-        const unsigned long long upto = ~0ull >> (63 - lr);  // positions 0..lr
-        int cnt = prior;  // entries starting before slot j's window
-#pragma unroll
-        for (int j = 0; j < PMAX; ++j) {
-            // clamped for slots past the chunk (int operands: a mixed
-            // int / unsigned max resolves to the double overload)
-            const int before = cnt + static_cast<int>(__popcll(w[j] & upto)) - 1;
-            e[j] = before > 0 ? before : 0;
-            cnt += static_cast<int>(__popcll(w[j]));
-        }
-        prior = cnt;
-        wave_sync();  // the bitmap is rewritten by the next round
-    } else {
-        int p[PMAX];
-#pragma unroll
-        for (int j = 0; j < PMAX; ++j) p[j] = base + j * L + lr;
-        chunk_find_all<EC, PMAX>(cm->off, p, e);
-    }
+    for (int j = 0; j < PMAX; ++j) p[j] = base + j * L + lr;
+    chunk_find_all<EC, PMAX>(cm->off, p, e);
     int at[PMAX];
 #pragma unroll
     for (int j = 0; j < PMAX; ++j) {
-        const int p = base + j * L + lr;
-        ok[j] = p < total;
-        // L == 64: d holds the entry's B position minus its product offset
-        at[j] = L == kWave ? p + cm->d[e[j]] : cm->d[e[j]] + p - cm->off[e[j]];
+        ok[j] = p[j] < total;
+        at[j] = cm->d[e[j]] + p[j] - cm->off[e[j]];
     }
     // The loads write registers that hold nothing else (no default to
     // merge with at the end of the branch, which would cost a copy and a
@@ -335,11 +268,9 @@ __device__ __forceinline__ void for_each_round(const GProb<V>& P, int a0, int a1
                 g(key, prod, ok);
             }
         } else {
-            int start[EC / L];
-            const int total = load_chunk<V, L, EC, VALS>(P, ebase, a1, lr, cm, s_tmp, start);
-            int prior = 0;
+            const int total = load_chunk<V, L, EC, VALS>(P, ebase, a1, lr, cm, s_tmp);
             for (int base = 0; base < total; base += L * PMAX) {
-                fetch_products<V, L, EC, PMAX, VALS>(P, cm, total, base, lr, start, prior, key, prod, ok);
+                fetch_products<V, L, EC, PMAX, VALS>(P, cm, total, base, lr, key, prod, ok);
                 g(key, prod, ok);
             }
             gsync<L>();  // the chunk metadata is overwritten next

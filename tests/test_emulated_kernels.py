@@ -367,12 +367,13 @@ SORTED = [(v, NUM[v][2]) for v in sorted(NUM) if NUM[v][0] == NUM[v][2] or (NUM[
 
 
 @pytest.mark.parametrize("variant,products", SORTED)
-@pytest.mark.parametrize("columns", [40, (1 << 25) - 1, 1 << 25, (1 << 26) - 1, 1 << 26])
+@pytest.mark.parametrize("columns", [40, 1 << 25, 1 << 26])
 def test_sorted_rows(emu, tmp_path, variant, products, columns):
     """Rows of one product up to the variant's slots and one more (a wave
     with such a row takes the hashed path), empty rows of B inside them,
-    repeated columns (40 columns), and column counts on both sides of the
-    limit that leaves room for the slot number beside the column."""
+    repeated columns (40 columns), and column counts at the limits that
+    leave no room for the slot number beside the column (2^25 for two
+    products a lane, 2^26 for one)."""
     rng = np.random.default_rng(variant)
     lens = [0, 1, 2, 3, 5, 7, 1, 4]
     pool = np.unique(np.r_[0, 1, columns - 1, rng.integers(0, columns, 40)])
@@ -394,6 +395,29 @@ def test_sorted_rows(emu, tmp_path, variant, products, columns):
     A, B = matrix(a_rows, 64, 95), matrix(b_rows, columns, 96)
     table = {1: f"{variant} {INT_MAX} {NUM[variant][2]}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
     run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A, B, "--f32", tables=table))
+
+
+@pytest.mark.parametrize("variant", [v["id"] for v in _NV if not v["global"] and v["lanes"] == 256 and v["chunk"] == 64])
+def test_group_rows_and_column_counts(emu, tmp_path, variant):
+    """Rows that the waves of a workgroup share, filled to one short of the
+    variant's capacity, with as many columns as leave room for the table
+    slot beside a sorted column (one fewer than 2^32 / slots) and one more,
+    where the slots are looked up again."""
+    _, _, p = NUM[variant]
+    limit = 2**32 // (2 * p)
+    table = {1: f"{variant} {INT_MAX} {p}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
+    rng = np.random.default_rng(variant)
+    calls = []
+    for n in (limit - 1, limit):
+        pool = np.sort(rng.choice(n - 2, p - 3, replace=False)) + 1
+        pool = np.r_[0, pool, n - 1]
+        b_rows = [pool[k::40] for k in range(40)] + [pool[:90]] * 3
+        rpt = np.concatenate([[0], np.cumsum([len(r) for r in b_rows])]).astype(np.int32)
+        col = np.concatenate(b_rows).astype(np.int32)
+        B = HostCSR(43, n, rpt, col, rng.uniform(-1, 1, col.size))
+        A = HostCSR(2, 43, np.array([0, 43, 63], np.int32), np.r_[0:43, 0:20].astype(np.int32), rng.uniform(-1, 1, 63))
+        calls.append(call(A, B, tables=table))
+    run_emu_all(emu, tmp_path, *calls)
 
 
 def test_batch_behind_a_product_without_entries(emu, tmp_path):
