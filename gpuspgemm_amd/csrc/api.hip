@@ -460,7 +460,7 @@ struct Context {
     BinTable sym{};
     BinTable num{};
     int occ_sym_multi = 1, occ_sym_max = 1;
-    int occ_num[2][kNumLdsVariants] = {};
+    int occ_num[2][kNumVariantCount] = {};
     // tiles from which the scan reads each tile's prefix off one scanned
     // array instead of summing the earlier tiles per workgroup (quadratic
     // in the tile count); SPG_TILE_PREFIX_MIN overrides it
@@ -508,7 +508,7 @@ void fill_table(BinTable& t, const TunedBin (&rows)[N], bool sym_phase) {
     for (int b = 0; b < t.n; ++b) {
         const int v = rows[b].variant;
         t.variant[b] = v;
-        t.rows[b] = sym_phase ? kSymVariants[v].r : (v < kNumGlobalVariant ? kNumVariants[v].r : 1);
+        t.rows[b] = sym_phase ? kSymVariants[v].r : kNumVariants[v].r;
         t.nip_cap[b] = rows[b].nip;
         t.nnz_cap[b] = rows[b].nnz;
     }
@@ -543,8 +543,8 @@ spg_status check_num_table(const BinTable& t) {
     if (t.n < 1 || t.n > kMaxBins) return fail(SPG_ERR_INVALID_ARGUMENT, "fused table: bad bin count");
     for (int b = 0; b < t.n; ++b) {
         const int v = t.variant[b];
-        if (v < 0 || v > kNumGlobalVariant) return fail(SPG_ERR_INVALID_ARGUMENT, "fused table: bad variant");
-        if (v < kNumGlobalVariant && (t.nnz_cap[b] > kNumVariants[v].p || t.nnz_cap[b] < 1))
+        if (v < 0 || v >= kNumVariantCount) return fail(SPG_ERR_INVALID_ARGUMENT, "fused table: bad variant");
+        if (v != kNumGlobalVariant && (t.nnz_cap[b] > kNumVariants[v].p || t.nnz_cap[b] < 1))
             return fail(SPG_ERR_INVALID_ARGUMENT, "fused table: nnz cap above the variant's capacity");
     }
     if (t.variant[t.n - 1] != kNumGlobalVariant || t.nnz_cap[t.n - 1] != INT_MAX || t.nip_cap[t.n - 1] != INT_MAX)
@@ -601,7 +601,7 @@ spg_status ensure_context(Context*& out) {
     c.occ_sym_max = occupancy_sym_max<double>();
     if (const char* env = std::getenv("SPG_TILE_PREFIX_MIN")) c.tile_prefix_min = std::max(1, std::atoi(env));
     if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::max(0, std::atoi(env));
-    for (int v = 0; v < kNumLdsVariants; ++v) {
+    for (int v = 0; v < kNumVariantCount; ++v) {
         c.occ_num[0][v] = occupancy_symnum_bin<float>(v);
         c.occ_num[1][v] = occupancy_symnum_bin<double>(v);
     }
@@ -1864,7 +1864,7 @@ static spg_status parse_table(int32_t phase, const char* text, BinTable& t) {
         if (phase == 0)
             t.rows[b] = (v >= 0 && v <= kSymMaxVariant) ? kSymVariants[v].r : 1;
         else
-            t.rows[b] = (v >= 0 && v < kNumGlobalVariant) ? kNumVariants[v].r : 1;
+            t.rows[b] = (v >= 0 && v < kNumVariantCount) ? kNumVariants[v].r : 1;
     }
     return phase == 0 ? check_sym_table(t) : check_num_table(t);
 }
@@ -1917,10 +1917,12 @@ spg_status spg_get_variants(int32_t phase, char* buf, size_t buf_len) {
                 << " chunk=" << kSymVariants[v].ec << " slots=" << kSymVariants[v].pmax
                 << (v == kSymMaxVariant ? " max" : "") << '\n';
     } else if (phase == 1) {
-        for (int v = 0; v < kNumGlobalVariant; ++v)
+        for (int v = 0; v < kNumVariantCount; ++v) {
+            if (v == kNumGlobalVariant) continue;
             out << v << " wg=" << kNumVariants[v].wg << " rows=" << kNumVariants[v].r << " capacity="
                 << kNumVariants[v].p << " chunk=" << kNumVariants[v].ec << " slots=" << kNumVariants[v].pmax
                 << (num_multi_set(v) >= 0 ? " merged=" + std::to_string(num_multi_set(v)) : std::string()) << '\n';
+        }
         out << kNumGlobalVariant << " global\n";
     } else {
         return fail(SPG_ERR_INVALID_ARGUMENT, "phase must be 0 or 1");

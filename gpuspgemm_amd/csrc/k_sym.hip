@@ -168,7 +168,7 @@ __device__ __forceinline__ void sym_units(const ProbSet<V>& ps, const int2* __re
             const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kLimit>(P, row, smem);
             if (threadIdx.x == 0) {
                 if (kLimit > 0 && n > kLimit)
-                    over_items[atomicAdd(&meta->over_count.v, 1)] = it;
+                    over_items[atomicAdd(&meta->fail_count.over, 1)] = it;
                 else
                     P.c_rpt[row] = n;
             }
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(1024) void k_sym_max(ProbSet<V> ps, const int2* __r
     constexpr SymVariant kV = kSymVariants[kSymMaxVariant];
     __shared__ __align__(16) int smem[sym_unit_lds<kSymMaxVariant>() / 4];
     const int2* bin_items = items + static_cast<long long>(bin) * bin_cap;
-    const int count = meta->sym_count[bin].v + meta->over_count.v;
+    const int count = meta->sym_count[bin].v + meta->fail_count.over;
     for (int u = blockIdx.x; u < count; u += gridDim.x) {
         const int2 it = bin_items[u];
         const GProb<V> P = ps.get(uniform(it.x));

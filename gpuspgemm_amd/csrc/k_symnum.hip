@@ -661,7 +661,7 @@ __global__ __launch_bounds__(kNumVariants[VV].wg) SPG_WAVES_PER_EU(kNumMinWaves[
 }
 
 #define SPG_NUM_VARIANTS(X) \
-    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(19) X(20)
+    X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16) X(17) X(18) X(20)
 
 // Several bins of the fused pass in one launch, a workgroup per unit.
 // Each XCD gets a contiguous slice of every bin (balanced work across the

@@ -191,14 +191,21 @@ struct alignas(128) Counter {
     T v;
 };
 
+// Rows that moved on during the count: `v` overflowed the largest table,
+// `over` were added to the last bin's list by its overflowing neighbour (both
+// rare, so they share a line).
+struct alignas(128) RowLists {
+    int32_t v;
+    int32_t over;
+};
+
 // Device counters of one multiply (zeroed by k_clear, or by the read-back
 // that ends the multiply before).  The second group
 // belongs to the scan / fused-bin stage and is cleared again on its own
 // when overflowed rows force that stage to run twice.
 struct DevMeta {
     Counter<int32_t> sym_count[kMaxBins];
-    Counter<int32_t> over_count;  // rows added to the last symbolic bin's list by its overflowing neighbour
-    Counter<int32_t> fail_count;
+    RowLists fail_count;
     Counter<int32_t> flags;
     Counter<int32_t> max_nip;
     Counter<unsigned long long> total_nip;

@@ -59,33 +59,34 @@ constexpr bool sym_is_wave(const SymVariant& v) { return v.wg / v.r == kWave; }
 constexpr bool sym_is_group(const SymVariant& v) { return v.wg / v.r > kWave; }
 
 // Fused sorted-columns + numeric variants, one kernel each: all use 256
-// threads except 9 (a 1024-thread workgroup per row); rows above every
-// capacity use global-memory tables (variant 21).  A row whose products fit
-// in one chunk and in lanes * pmax keeps them in registers between the two
-// halves.  Variants 10..18 cover the small capacities with 2 to 32 lanes
-// per row; the tuner picks among them per bin.
+// threads except 9 and 20 (a 1024-thread workgroup per row); rows above every
+// capacity use global-memory tables (variant 19).  4, 5 and 13: a row to a
+// wave; 6 and 7: a row to a workgroup's waves, values in the table; 20: the
+// longest rows, columns in LDS; 8 and 9: a row to a workgroup in step, with
+// searches in the sorted list; the others several rows to a wave.  10 to 13
+// (and 5) sort rows with a product per lane (two) in registers.  The tuner
+// picks among those that fit a bin.
 constexpr NumVariant kNumVariants[] = {
     {256, 256, 8, 4, 16},   {256, 128, 16, 4, 16}, {256, 64, 32, 8, 16},  {256, 32, 64, 16, 16},
-    {256, 16, 128, 32, 16}, {256, 4, 128, 64, 4, 256}, {256, 4, 256, 64, 4, 512}, {256, 1, 1024, 64, 4, 2048},
-    {256, 1, 512, 64, 4, 1024}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
+    {256, 4, 256, 64, 4, 512}, {256, 4, 128, 64, 4, 256}, {256, 1, 512, 64, 4, 1024}, {256, 1, 1024, 64, 4, 2048},
+    {256, 1, 2048, 256, 8}, {1024, 1, 8192, 1024, 4}, {256, 32, 8, 8, 2}, {256, 16, 16, 16, 2},
     {256, 8, 32, 32, 4},    {256, 4, 64, 64, 4, 128}, {256, 64, 8, 8, 4},    {256, 128, 8, 4, 8},
-    {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},  {256, 1, 2048, 256, 8},
+    {256, 32, 16, 8, 4},    {256, 64, 16, 8, 8},   {256, 32, 32, 16, 8},  {1024, 1, 1, 1, 1},
     {1024, 1, 26214, 64, 4, 32768},
 };
-constexpr int kNumLdsVariants = 21;  // variants with an LDS kernel (0..20)
+constexpr int kNumVariantCount = 21;
+constexpr int kNumGlobalVariant = 19;  // (its entry above only holds the place)
 // Waves per SIMD that each fused variant's kernel must keep (its register
-// budget is 512 / waves VGPRs).  Fetching a lane's products as one batch
-// of loads (every load in flight before the first multiply) needs more
-// registers than fetching them one by one; the floor keeps the residency
-// the variant had with the one-by-one fetch, and the compiler schedules
-// the batch within it.  Measured on gfx950: the 96^3 stencil's fused pass
-// 3.23 -> 2.81 ms, the power-law's 198k-row bin 70 -> 53 us.
-constexpr int kNumMinWaves[kNumLdsVariants] = {3, 3, 3, 3, 3, 8, 5, 5, 8, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 3, 4};
-constexpr int kNumGlobalVariant = 21;
+// budget is 512 / waves VGPRs).  The floors of the narrow variants keep the
+// residency that they had when a lane's products were fetched one by one
+// (power-law: 198k-row bin 70 -> 53 us with the batch inside it); the wave
+// rows' eight waves (64 VGPRs) beat six by 7 % (96^3 stencil).
+constexpr int kNumMinWaves[kNumVariantCount] = {3, 3, 3, 3, 5, 8, 8, 5, 3, 4, 8, 8, 7, 8, 7, 5, 7, 5, 5, 1, 4};
 
 // Fused variants whose bins share one launch.  Set 0, small rows (256
-// threads, up to 32 lanes per row, about 64 VGPRs): their bins hold most
-// rows of skewed matrices, and one launch keeps the GPU filled across them
+// threads, up to a wave per row, about 78 VGPRs; floors of seven and eight
+// waves measured +4 and +1 % on the power-law, -2 and -3 % on a batch):
+// their bins hold most rows of skewed matrices, and one launch keeps the GPU filled across them
 // where separate launches would queue behind each other on the lane's few
 // hardware queues.  Set 1, the 256-thread variants of longer rows: merged
 // only while their bins are small (a few thousand units, as the heavy tail
@@ -153,7 +154,7 @@ constexpr int max_sym_multi_lds() {
 }
 constexpr int max_num_lds() {
     int m = 0;
-    for (int i = 0; i < kNumLdsVariants; ++i) {
+    for (int i = 0; i < kNumVariantCount; ++i) {
         const int b = 4 * kNumVariants[i].r * num_row_ints(kNumVariants[i]);
         m = m > b ? m : b;
     }
@@ -161,7 +162,7 @@ constexpr int max_num_lds() {
 }
 constexpr int max_num_multi_lds(int set) {
     int m = 0;
-    for (int v = 0; v < kNumLdsVariants; ++v) {
+    for (int v = 0; v < kNumVariantCount; ++v) {
         const int b = 4 * kNumVariants[v].r * num_row_ints(kNumVariants[v]);
         if (num_multi_set(v) == set) m = m > b ? m : b;
     }
