@@ -276,12 +276,6 @@ __device__ __forceinline__ int table_insert_from(int* tab, int key, uint32_t h, 
     }
 }
 
-template <int T>
-__device__ __forceinline__ int table_insert(int* tab, int key) {
-    const uint32_t h = hash_slot<T>(key);
-    return table_insert_from<T>(tab, key, h, lds_load(tab + h));
-}
-
 // Insert up to N staged keys: the first probes of all keys are read
 // together (independent LDS loads), then each key finishes its probe.
 template <int T, int N>
