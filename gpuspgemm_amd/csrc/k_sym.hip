@@ -75,16 +75,19 @@ __device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* 
 #pragma unroll
         for (int i = 0; i < T / (4 * kWave); ++i)
             reinterpret_cast<Words*>(tab)[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
-        const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide) != 0};
+        const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr,
+                                uniform(P.wide) != 0, far_columns(uniform(P.n))};
         wave_sync();
         const int inst_next = uniform(it_next.x), row_next = uniform(it_next.y);
         const GProb<V> P_next = ps.get(inst_next);
         const int b0 = P_next.a_rpt[row_next], b1 = P_next.a_rpt[row_next + 1];
         int n = 0;
-        wave_products<V, N, false>(W, a0, a1, walk, [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) {
-            uint32_t h[N];
-            table_slots<T, N, true>(tab, key, ok, h, n);
-        });
+        wave_products<V, N, false>(
+            W, a0, a1, walk,
+            [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N], auto far) {
+                uint32_t h[N];
+                table_slots<T, far, N, true>(tab, key, ok, h, n);
+            });
         if (lane == 0) P.c_rpt[row] = n;
         if (!more) break;
         wave_sync();  // the table is reused by the next row
@@ -114,7 +117,8 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
     for (int i = 0; i < T / (4 * WG); ++i)
         reinterpret_cast<Words*>(tab)[i * WG + threadIdx.x] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
     if (threadIdx.x == 0) *total = 0;
-    const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide) != 0};
+    const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr,
+                                uniform(P.wide) != 0, far_columns(uniform(P.n))};
     const int a0 = uniform(P.a_rpt[row]), a1 = uniform(P.a_rpt[row + 1]);
     const int nip = uniform(P.nip[row]);
     __syncthreads();
@@ -125,12 +129,12 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
     };
     wave_products<V, N, false>(
         W, a0, a1, walk + wave,
-        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) -> bool {
+        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N], auto far) -> bool {
             if constexpr (LIMIT > 0) {
                 if (uniform(lds_load(total)) > LIMIT) return false;
             }
             uint32_t h[N];
-            table_slots<T, N, true>(tab, key, ok, h, added);
+            table_slots<T, far, N, true>(tab, key, ok, h, added);
             if constexpr (LIMIT > 0) report();
             return true;
         },

@@ -105,7 +105,7 @@ __device__ __forceinline__ void symnum_sorted(const GProb<V>& Pr, const RowItem&
     const int lane = lane_id();
     const int lr = lane % L;
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), false};
+                            uniform_ptr(Pr.b_val), false, false};
     const auto c_col = uniform_ptr(Pr.c_col);
     const auto c_val = uniform_ptr(Pr.c_val);
     if (lane < K) sl.starts[lane] = 0;
@@ -357,17 +357,18 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
             v[i * kWave + lane] = Words{0, 0, 0, 0};
     }
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
     wave_sync();
-    wave_products<V, N, true>(W, uniform(it.a0), uniform(it.a1), &row.walk,
-                              [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
-                                  uint32_t h[N];
-                                  int fresh = 0;
-                                  table_slots<T>(row.keys, key, ok, h, fresh);
+    wave_products<V, N, true>(
+        W, uniform(it.a0), uniform(it.a1), &row.walk,
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N], auto far) {
+            uint32_t h[N];
+            int fresh = 0;
+            table_slots<T, far>(row.keys, key, ok, h, fresh);
 #pragma unroll
-                                  for (int j = 0; j < N; ++j)
-                                      if (in_mask(ok[j])) lds_add(row.vals + h[j], prod[j]);
-                              });
+            for (int j = 0; j < N; ++j)
+                if (in_mask(ok[j])) lds_add(row.vals + h[j], prod[j]);
+        });
     wave_sync();
 
     // the occupied slots, S consecutive ones to a lane, in front of each other
@@ -441,15 +442,15 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     const RowItem it = load_item(items, idx);
     const GProb<V> Pr = ps.get(uniform(it.inst));
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
     const int a0 = uniform(it.a0), a1 = uniform(it.a1);
     __syncthreads();
     wave_products<V, N, true>(
         W, a0, a1, &row.walk[wave],
-        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N], auto far) {
             uint32_t h[N];
             int fresh = 0;
-            table_slots<T>(row.keys, key, ok, h, fresh);
+            table_slots<T, far>(row.keys, key, ok, h, fresh);
 #pragma unroll
             for (int j = 0; j < N; ++j)
                 if (in_mask(ok[j])) lds_add(row.vals + h[j], prod[j]);
@@ -548,7 +549,7 @@ __device__ __forceinline__ void symnum_long_row(const ProbSet<V>& ps, const RowI
     const RowItem it = load_item(items, idx);
     const GProb<V> Pr = ps.get(uniform(it.inst));
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
     const int a0 = uniform(it.a0), a1 = uniform(it.a1), cn = uniform(it.cn);
     const bool by_chunk = wave_by_chunk<kWaves>(a1 - a0, uniform(it.nip));
     const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);
@@ -558,10 +559,10 @@ __device__ __forceinline__ void symnum_long_row(const ProbSet<V>& ps, const RowI
     // (the walk without values uses the front of the same metadata)
     wave_products<V, N, false>(
         W, a0, a1, reinterpret_cast<WaveChunk<false>*>(&row.walk[wave]),
-        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N]) {
+        [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N], auto far) {
             uint32_t h[N];
             int fresh = 0;
-            table_slots<T>(row.keys, key, ok, h, fresh);
+            table_slots<T, far>(row.keys, key, ok, h, fresh);
         },
         wave, kWaves, by_chunk);
     __syncthreads();
@@ -602,7 +603,7 @@ __device__ __forceinline__ void symnum_long_row(const ProbSet<V>& ps, const RowI
     const int half = n <= T / 2 ? T / 4 : T / 2;
     wave_products<V, N, true>(
         W, a0, a1, &row.walk[wave],
-        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N]) {
+        [&](const int(&key)[N], const LdsSum(&prod)[N], const unsigned long long(&ok)[N], auto far) {
             int pos[N];
 #pragma unroll
             for (int j = 0; j < N; ++j) pos[j] = 0;

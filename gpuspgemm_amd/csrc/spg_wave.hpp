@@ -51,9 +51,11 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 // The value of lane 63.
 __device__ __forceinline__ int wave_last(int v) { return __builtin_amdgcn_readlane(v, kWave - 1); }
 
-// Slot of a column in a table of T <= 2^16 slots: the fraction of
-// column * golden ratio, from the low 24 bits of both factors (columns that
-// differ by a multiple of 2^24 share a slot and probe on).
+// Slot of a column below 2^24 in a table of T <= 2^16 slots: the fraction of
+// column * golden ratio, from the low 24 bits of both factors.  Matrices of
+// more columns (FAR) take hash_slot: here columns that differ by a multiple of
+// 2^24 would share a slot, and 20,000 rows of 27 x 27 products on columns 2^24
+// apart took 5.9 ms instead of 0.12 (2^20 apart: 1.4 instead of 0.32).
 template <int T>
 __device__ __forceinline__ uint32_t slot24(int key) {
     constexpr int kBits = __builtin_ctz(T);
@@ -69,6 +71,16 @@ __device__ __forceinline__ uint32_t slot24(int key) {
     return (x >> (24 - kBits)) & (T - 1);
 }
 
+// Whether a matrix has columns that slot24 does not tell apart.
+__device__ __forceinline__ bool far_columns(int columns) { return columns > 1 << 24; }
+template <int T, bool FAR>
+__device__ __forceinline__ uint32_t walk_slot(int key) {
+    if constexpr (FAR)
+        return hash_slot<T>(key);
+    else
+        return slot24<T>(key);
+}
+
 // Slots of N keys in an LDS table of T slots (open addressing, linear
 // probing), inserting those that are new; ok[j]: the lanes that have a key j.
 // The probes of all keys advance together, each a compare-and-swap.  Lane
@@ -77,14 +89,14 @@ __device__ __forceinline__ uint32_t slot24(int key) {
 // instruction), and a key whose lanes are all done costs nothing more.
 // The table never fills (its row has fewer distinct columns than T).  With
 // COUNT, `fresh` grows by the number of keys the wave inserted.
-template <int T, int N, bool COUNT = false>
+template <int T, bool FAR, int N, bool COUNT = false>
 __device__ __forceinline__ void table_slots(int* tab, const int (&key)[N], const unsigned long long (&ok)[N],
                                             uint32_t (&h)[N], int& fresh) {
     int old[N];
     unsigned long long pend[N], any = 0;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-        h[j] = slot24<T>(key[j]);
+        h[j] = walk_slot<T, FAR>(key[j]);
         if (in_mask(ok[j])) old[j] = atomicCAS(tab + h[j], kEmpty, key[j]);
     }
 #pragma unroll
@@ -122,8 +134,9 @@ struct SlotWord {
     static constexpr int kBits = __builtin_ctz(T);
     int shift;       // scalar: kBits or 0
     uint32_t slots;  // scalar: T - 1 or 0
+    bool far;        // scalar: far_columns
     __device__ __forceinline__ explicit SlotWord(int columns)
-        : shift(columns < (1 << (32 - kBits)) ? kBits : 0), slots(shift ? T - 1 : 0) {}
+        : shift(columns < (1 << (32 - kBits)) ? kBits : 0), slots(shift ? T - 1 : 0), far(far_columns(columns)) {}
     __device__ __forceinline__ uint32_t pack(int key, int slot) const {
         return static_cast<uint32_t>(key) << shift | (static_cast<uint32_t>(slot) & slots);
     }
@@ -133,14 +146,14 @@ struct SlotWord {
 
 // Slot of a key that is in the table.
 template <int T>
-__device__ __forceinline__ uint32_t table_find(const int* tab, int key) {
-    uint32_t h = slot24<T>(key);
+__device__ __forceinline__ uint32_t table_find(const int* tab, int key, bool far) {
+    uint32_t h = far ? walk_slot<T, true>(key) : walk_slot<T, false>(key);
     while (lds_load(tab + h) != key) h = (h + 1) & (T - 1);
     return h;
 }
 template <int T>
 __device__ __forceinline__ uint32_t SlotWord<T>::slot(const int* tab, uint32_t w) const {
-    return shift ? w & (T - 1) : table_find<T>(tab, static_cast<int>(w));
+    return shift ? w & (T - 1) : table_find<T>(tab, static_cast<int>(w), far);
 }
 
 // Sort of 64 * E keys, lane l holding keys l*E .. l*E + E-1 of the result
@@ -355,10 +368,12 @@ struct WaveOperands {
     const int32_t SPG_GLOBAL* b_col;
     const V SPG_GLOBAL* b_val;
     bool wide;  // B's arrays may pass 4 GiB: 64-bit offsets
+    bool far;   // far_columns of B
 };
 
 // The products of A's entries [a0, a1), in rounds of N * 64:
-// f(key[N], prod[N], ok[N]), ok[j] the lanes with a product j.  The wave takes 64 entries at a time, one to a
+// f(key[N], prod[N], ok[N], far), ok[j] the lanes with a product j, far the
+// constant FAR (far_columns of B).  The wave takes 64 entries at a time, one to a
 // lane; entries with an empty row of B drop out.  A product's entry is the
 // number of entries that start at or before it (less one): the chunk's
 // starts are marked in a bitmap, 64 products to a word and one position
@@ -368,7 +383,7 @@ struct WaveOperands {
 // ... of every window, or, with `by_chunk`, every round of the chunks first,
 // first + step, ... instead.  An f that
 // returns false (the same on every lane) ends the walk.
-template <typename V, int N, bool VALS, bool WIDE, typename F>
+template <typename V, int N, bool VALS, bool WIDE, bool FAR, typename F>
 __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                                  int first, int step, bool by_chunk) {
     static_assert(N <= kWavePad, "a round may pass the window by N - 1 words");
@@ -454,10 +469,11 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
 #pragma unroll
                     for (int j = 0; j < N; ++j) prod[j] = a[j] * static_cast<LdsSum>(bv[j]);
                 }
-                if constexpr (std::is_same_v<decltype(f(key, prod, ok)), bool>) {
-                    if (!f(key, prod, ok)) return;
+                constexpr std::bool_constant<FAR> far{};
+                if constexpr (std::is_same_v<decltype(f(key, prod, ok, far)), bool>) {
+                    if (!f(key, prod, ok, far)) return;
                 } else {
-                    f(key, prod, ok);
+                    f(key, prod, ok, far);
                 }
             }
         }
@@ -467,10 +483,13 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
 template <typename V, int N, bool VALS, typename F>
 __device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                               int first = 0, int step = 1, bool by_chunk = true) {
+    // (a copy of the walk each: chosen round by round instead, the hash cost the 96^3 stencil 5 %)
     if (W.wide)
-        wave_products_at<V, N, VALS, true>(W, a0, a1, wc, f, first, step, by_chunk);
+        wave_products_at<V, N, VALS, true, true>(W, a0, a1, wc, f, first, step, by_chunk);
+    else if (W.far)
+        wave_products_at<V, N, VALS, false, true>(W, a0, a1, wc, f, first, step, by_chunk);
     else
-        wave_products_at<V, N, VALS, false>(W, a0, a1, wc, f, first, step, by_chunk);
+        wave_products_at<V, N, VALS, false, false>(W, a0, a1, wc, f, first, step, by_chunk);
 }
 
 // How the waves of a workgroup share a row: by chunks of 64 entries when

@@ -325,6 +325,14 @@ void drain_blocking() {
     });
 }
 
+// EMU_COUNT_CAS=1 prints the number of compare-and-swaps of all kernels at
+// the end: with linear probing, how far keys lie from their slots.
+static const struct CasReport {
+    ~CasReport() {
+        if (std::getenv("EMU_COUNT_CAS")) std::printf("compare-and-swaps %llu\n", cas_count.load());
+    }
+} g_cas_report;
+
 int lane() { return static_cast<int>(tl_thread.x % 64); }
 void block_barrier() {
     g_wave_bar[tl_thread.x / 64].park(1);

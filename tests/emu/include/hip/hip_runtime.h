@@ -231,7 +231,11 @@ inline int atomicAdd(int* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_S
 inline unsigned long long atomicAdd(unsigned long long* p, unsigned long long v) {
     return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST);
 }
+namespace emu {
+inline std::atomic<unsigned long long> cas_count{0};  // compare-and-swaps of all kernels so far
+}
 inline int atomicCAS(int* p, int cmp, int val) {
+    emu::cas_count.fetch_add(1, std::memory_order_relaxed);
     __atomic_compare_exchange_n(p, &cmp, val, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
     return cmp;
 }

@@ -420,6 +420,37 @@ def test_group_rows_and_column_counts(emu, tmp_path, variant):
     run_emu_all(emu, tmp_path, *calls)
 
 
+# one variant of every kind of row that looks columns up with table_slots: a
+# wave, a workgroup, and (fused) a long row's workgroup
+PROBED = [(0, min(v for v in SYM if SYM[v][0] == 64)), (0, max(v for v in SYM if SYM[v][0] == 256)),
+          (1, min(v for v in NUM if NUM[v][0] == 64)), (1, min(v for v in NUM if NUM[v][:2] == (256, 64))),
+          (1, max(v for v in NUM if NUM[v][:2] == (1024, 64)))]
+
+
+@pytest.mark.parametrize("phase,variant", PROBED)
+def test_columns_far_apart(emu, tmp_path, phase, variant):
+    """Columns that lie a large power of two apart (as the block indices of a
+    flattened tensor) must not share table slots: a product on 64 columns
+    2^20 apart takes at most half as many compare-and-swaps again as the
+    same product on adjacent columns."""
+    if phase == 0:
+        table = {0: f"{variant} {SYM[variant][2] // 2 - 1} {INT_MAX}\n{SYM_MAX} {INT_MAX} {INT_MAX}\n"}
+    else:
+        table = {1: f"{variant} {INT_MAX} {NUM[variant][2]}\n{NUM_GLOBAL} {INT_MAX} {INT_MAX}\n"}
+    count, stride = 64, 1 << 20
+    rng = np.random.default_rng(variant)
+    k = 40
+    B = HostCSR(6, count, (np.arange(7) * k).astype(np.int32),
+                np.concatenate([np.sort(rng.choice(count, k, replace=False)) for _ in range(6)]).astype(np.int32),
+                rng.uniform(-1, 1, 6 * k))
+    far = HostCSR(6, (count - 1) * stride + 1, B.rpt, B.col * np.int32(stride), B.val)
+    A = HostCSR(2, 6, np.array([0, 6, 11], np.int32), np.r_[0:6, 1:6].astype(np.int32), rng.uniform(-1, 1, 11))
+    env = {"EMU_COUNT_CAS": "1"}
+    out = run_emu_all(emu, tmp_path, call(A, B, tables=table, env=env), call(A, far, tables=table, env=env))
+    near_cas, far_cas = (int(o.split("compare-and-swaps ")[1].split()[0]) for o in out)
+    assert far_cas <= 1.5 * near_cas, (near_cas, far_cas)
+
+
 def test_batch_behind_a_product_without_entries(emu, tmp_path):
     """A batch whose first product has no entries (null arrays): a wave of a
     fused unit that has no row sees item zero, instance zero, and must not
