@@ -326,11 +326,12 @@ def test_wave_rows_count_entry_starts(emu, tmp_path, phase, variant):
                 call(A.astype(np.float32), B.astype(np.float32), "--f32", tables=table))
 
 
-def _heavy_row_case():
-    """A row that overflows the largest LDS table in the count pass and every
-    LDS capacity in the fused pass, plus three ordinary rows."""
+def _heavy_row_case(draws=9500):
+    """A row of 21,525 columns, among the longest that the largest LDS tables
+    of both passes hold (16,000 draws: 30,427, more than they hold), plus
+    three ordinary rows."""
     nb = 20_000
-    r0 = np.unique(gen.rand_below(3, 1, np.arange(9500), np.full(9500, nb)))
+    r0 = np.unique(gen.rand_below(3, 1, np.arange(draws), np.full(draws, nb)))
     rows = [r0] + [np.unique(gen.rand_below(3, 3 + i, np.arange(3), np.full(3, nb))) for i in range(3)]
     rpt = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
     col = np.concatenate(rows).astype(np.int32)
@@ -489,10 +490,26 @@ def test_symbolic_overflow_moves_to_the_largest_table(emu, tmp_path):
 
 
 def test_global_paths(emu, tmp_path):
-    """The heavy-row case first with the default tables and then with every
-    row forced to the global kernels."""
+    """The heavy-row case first with the default tables, a long row of the
+    largest LDS variants, and then with every row forced to the global
+    kernels."""
     A, B = _heavy_row_case()
+    longest = max(p for _, _, p in NUM.values())
+    assert 16384 < int(np.diff(oracle.spgemm(A, B).rpt).max()) <= longest
     run_emu_all(emu, tmp_path, call(A, B), call(A, B, tables=GLOBAL_TABLES))
+
+
+def test_row_past_the_largest_tables(emu, tmp_path):
+    """A row of more columns than the largest count table admits: its waves
+    stop, it joins the overflow list, is counted again in global memory (a
+    second scan follows) and takes the global fused kernel, with the default
+    tables."""
+    A, B = _heavy_row_case(draws=16_000)
+    assert int(np.diff(oracle.spgemm(A, B).rpt).max()) > max(p for _, _, p in NUM.values())
+    out = run_emu(emu, tmp_path, A, B, env={"SPG_LOG_LEVEL": "debug"})
+    line = next(x for x in out.splitlines() if "symbolic phase" in x)
+    assert "fail bin 1," in line, line
+    assert line.split("rows per fused bin [")[1].split("]")[0].split()[-1] == "1", line
 
 
 def test_noalloc_entry(emu, tmp_path):
