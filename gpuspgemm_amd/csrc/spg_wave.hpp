@@ -380,15 +380,16 @@ struct WaveOperands {
 // early, so that a lane counts the marks below its own bit (two mbcnt on
 // top of the count before the word).  `first` and `step` let
 // several waves share a row: this wave takes the rounds first, first + step,
-// ... of every window, or, with `by_chunk`, every round of the chunks first,
-// first + step, ... instead.  An f that
+// ... of the row, counted on over its windows and chunks, or, with `by_chunk`,
+// every round of the chunks first, first + step, ... instead.  An f that
 // returns false (the same on every lane) ends the walk.
 template <typename V, int N, bool VALS, bool WIDE, bool FAR, typename F>
 __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                                  int first, int step, bool by_chunk) {
     static_assert(N <= kWavePad, "a round may pass the window by N - 1 words");
     const int lane = lane_id();
-    const int round0 = by_chunk ? 0 : first, round_step = by_chunk ? 1 : step;
+    const int round_step = by_chunk ? 1 : step;
+    int r = by_chunk ? 0 : first;  // this wave's next round, from the window's first on
     for (int ebase = a0 + (by_chunk ? first * kWave : 0); ebase < a1; ebase += by_chunk ? step * kWave : kWave) {
         const int e = ebase + lane;
         long long ref = 0;
@@ -410,6 +411,12 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
             wc->ent[rank_in(filled)] = w;
         }
         for (int win = 0; win < total; win += kWave * kWaveWords) {
+            const int in_win = min(total - win, kWave * kWaveWords);
+            const int n_rounds = (in_win + N * kWave - 1) / (N * kWave);
+            if (r >= n_rounds) {  // the other waves' rounds
+                r -= n_rounds;
+                continue;
+            }
             wave_sync();  // the previous window's reads are done
             if (lane < kWaveWords + kWavePad) wc->starts[lane] = 0;
             wave_sync();
@@ -425,9 +432,7 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
                 if (lane < kWaveWords + kWavePad) wc->before[lane] = earlier + up - c;
             }
             wave_sync();
-            const int in_win = min(total - win, kWave * kWaveWords);
-            const int n_rounds = (in_win + N * kWave - 1) / (N * kWave);
-            for (int r = round0; r < n_rounds; r += round_step) {
+            for (; r < n_rounds; r += round_step) {
                 const int base = r * N * kWave;  // in the window
                 int en[N];
 #pragma unroll
@@ -476,6 +481,7 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
                     f(key, prod, ok, far);
                 }
             }
+            r -= n_rounds;
         }
     }
 }
@@ -492,12 +498,20 @@ __device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, 
         wave_products_at<V, N, VALS, false, false>(W, a0, a1, wc, f, first, step, by_chunk);
 }
 
-// How the waves of a workgroup share a row: by chunks of 64 entries when
-// every wave gets one and the rows of B are short (a chunk is then a few
-// rounds), otherwise round by round, each wave reading every chunk.
+// How the waves of a workgroup share a row: by chunks of 64 entries, or by
+// rounds, for which every wave reads every chunk.  Reading a chunk takes a
+// wave about as long as two rounds of 256 products, so chunks are dealt where
+// the busiest wave's share of them, with their rounds, is the shorter.
 template <int WAVES>
 __device__ __forceinline__ bool wave_by_chunk(int entries, int nip) {
-    return entries >= WAVES * kWave && nip / 16 < entries;
+    constexpr int kRead = 2;  // rounds that take as long as reading a chunk
+    if (entries <= kWave) return false;
+    if (entries >= 8 * WAVES * kWave) return true;
+    const int chunks = (entries + kWave - 1) / kWave;
+    const int share = (chunks + WAVES - 1) / WAVES;
+    const int rounds = nip / (4 * kWave) + chunks;
+    // share * (kRead + rounds / chunks) < kRead * chunks + rounds / WAVES
+    return rounds * (share * WAVES - chunks) < kRead * WAVES * chunks * (chunks - share);
 }
 
 }  // namespace spg

@@ -421,6 +421,49 @@ def test_group_rows_and_column_counts(emu, tmp_path, variant):
     run_emu_all(emu, tmp_path, *calls)
 
 
+@pytest.fixture(scope="module")
+def wave_share():
+    exe = os.path.join(BUILD, "wave_share")
+    tmp = f"{exe}.{os.getpid()}"
+    os.makedirs(BUILD, exist_ok=True)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address", "-pthread", "-I",
+                    os.path.join(EMU, "include"), "-I", CSRC, os.path.join(EMU, "wave_share.cpp"),
+                    os.path.join(EMU, "emu_runtime.cpp"), "-o", tmp], check=True)
+    os.replace(tmp, exe)
+    return exe
+
+
+@pytest.mark.parametrize("waves", [4, 16])
+@pytest.mark.parametrize("entries,b_row", [(40, 3), (64, 5), (130, 4), (250, 3), (733, 4), (300, 9), (300, 20),
+                                           (60, 60), (1030, 2), (90, 40)])
+def test_waves_share_a_row_evenly(wave_share, waves, entries, b_row):
+    """The waves of a workgroup walk a row together (by rounds, by chunks of
+    64 entries, and as the rule picks): every product goes to one wave
+    once; dealt by rounds, the waves' round counts differ by at most one,
+    with one, two or three rounds to a chunk as with many; and the busiest
+    wave's chunks read and rounds, as the rule weighs them, are no more
+    than in the better of the two ways."""
+    out = subprocess.run([wave_share, str(waves), str(entries), str(b_row)], stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout
+    cost = {}
+    for line in out.stdout.splitlines():
+        how, rounds, hits = line.split(":")
+        rounds = [int(x) for x in rounds.split()]
+        assert len(rounds) == waves and hits.split() == ["1", "1"], line
+        if how != "rule":
+            chunks = -(-entries // 64)
+            cost[how] = max(rounds) + 2 * (chunks if how == "rounds" else -(-chunks // waves))
+        if how == "rounds":
+            assert max(rounds) - min(rounds) <= 1, line
+        if how == "rule":
+            picked = rounds
+    by = {line.split(":")[0]: [int(x) for x in line.split(":")[1].split()] for line in out.stdout.splitlines()}
+    best = min(cost.values())
+    # (the rule rounds the average up: one round more is as good)
+    assert any(picked == by[how] and cost[how] <= best + 1 for how in cost), (cost, out.stdout)
+
+
 # one variant of every kind of row that looks columns up with table_slots: a
 # wave, a workgroup, and (fused) a long row's workgroup
 PROBED = [(0, min(v for v in SYM if SYM[v][0] == 64)), (0, max(v for v in SYM if SYM[v][0] == 256)),
