@@ -1101,7 +1101,7 @@ struct Job : JobBase {
             p.bref = bref + entry_base;
             p.m = A[i].m;
             p.n = B[i].n;
-            p.wide = B[i].nnz >= c.wide_min ? 1 : 0;
+            p.wide = (B[i].nnz >= c.wide_min ? kWideOffsets : 0) | (B[i].n > 1 << 24 ? kWideColumns : 0);
             if (batch) {
                 const int first = static_cast<int>(tiles.size());
                 for (int r0 = 0; r0 < A[i].m; r0 += kTileRows)

@@ -75,8 +75,7 @@ __device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* 
 #pragma unroll
         for (int i = 0; i < T / (4 * kWave); ++i)
             reinterpret_cast<Words*>(tab)[i * kWave + lane] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
-        const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr,
-                                uniform(P.wide) != 0, far_columns(uniform(P.n))};
+        const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide)};
         wave_sync();
         const int inst_next = uniform(it_next.x), row_next = uniform(it_next.y);
         const GProb<V> P_next = ps.get(inst_next);
@@ -117,8 +116,7 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
     for (int i = 0; i < T / (4 * WG); ++i)
         reinterpret_cast<Words*>(tab)[i * WG + threadIdx.x] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
     if (threadIdx.x == 0) *total = 0;
-    const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr,
-                                uniform(P.wide) != 0, far_columns(uniform(P.n))};
+    const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide)};
     const int a0 = uniform(P.a_rpt[row]), a1 = uniform(P.a_rpt[row + 1]);
     const int nip = uniform(P.nip[row]);
     __syncthreads();

@@ -105,7 +105,7 @@ __device__ __forceinline__ void symnum_sorted(const GProb<V>& Pr, const RowItem&
     const int lane = lane_id();
     const int lr = lane % L;
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), false, false};
+                            uniform_ptr(Pr.b_val), 0};
     const auto c_col = uniform_ptr(Pr.c_col);
     const auto c_val = uniform_ptr(Pr.c_val);
     if (lane < K) sl.starts[lane] = 0;
@@ -209,8 +209,8 @@ __device__ __forceinline__ void symnum_sorted(const GProb<V>& Pr, const RowItem&
 // Whether symnum_sorted takes a wave's rows (every lane: its row's item).
 template <typename V, int L, int K>
 __device__ __forceinline__ bool sorted_fits(const GProb<V>& Pr, const RowItem& it, bool active) {
-    const bool fits = it.nip <= L * K && it.a1 - it.a0 <= L && it.inst == uniform(it.inst) && !Pr.wide &&
-                      Pr.n < 1 << kSortColBits<K>;
+    const bool fits = it.nip <= L * K && it.a1 - it.a0 <= L && it.inst == uniform(it.inst) &&
+                      !(Pr.wide & kWideOffsets) && Pr.n < 1 << kSortColBits<K>;
     return __ballot(active && !fits) == 0;
 }
 
@@ -357,7 +357,7 @@ __device__ __forceinline__ void symnum_wave_row(const ProbSet<V>& ps, const RowI
             v[i * kWave + lane] = Words{0, 0, 0, 0};
     }
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide)};
     wave_sync();
     wave_products<V, N, true>(
         W, uniform(it.a0), uniform(it.a1), &row.walk,
@@ -442,7 +442,7 @@ __device__ __forceinline__ void symnum_group_row(const ProbSet<V>& ps, const Row
     const RowItem it = load_item(items, idx);
     const GProb<V> Pr = ps.get(uniform(it.inst));
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide)};
     const int a0 = uniform(it.a0), a1 = uniform(it.a1);
     __syncthreads();
     wave_products<V, N, true>(
@@ -549,7 +549,7 @@ __device__ __forceinline__ void symnum_long_row(const ProbSet<V>& ps, const RowI
     const RowItem it = load_item(items, idx);
     const GProb<V> Pr = ps.get(uniform(it.inst));
     const WaveOperands<V> W{uniform_ptr(Pr.a_val), uniform_ptr(Pr.bref), uniform_ptr(Pr.b_col),
-                            uniform_ptr(Pr.b_val), uniform(Pr.wide) != 0, far_columns(uniform(Pr.n))};
+                            uniform_ptr(Pr.b_val), uniform(Pr.wide)};
     const int a0 = uniform(it.a0), a1 = uniform(it.a1), cn = uniform(it.cn);
     const bool by_chunk = wave_by_chunk<kWaves>(a1 - a0, uniform(it.nip));
     const auto ccol = uniform_ptr(Pr.c_col) + uniform(it.c0);

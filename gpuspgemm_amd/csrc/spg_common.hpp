@@ -55,7 +55,11 @@ struct Prob {
     long long* bref;
     int32_t m;
     int32_t n;
-    int32_t wide;  // B's columns or values may reach past 4 GiB: byte offsets need 64 bits
+    int32_t wide;  // kWideOffsets, kWideColumns
+};
+enum WideFlags : int32_t {
+    kWideOffsets = 1,  // B's columns or values may reach past 4 GiB: byte offsets need 64 bits
+    kWideColumns = 2,  // B has more than 2^24 columns: the hash needs 32 bits
 };
 
 // An entry's row of B packed in one word: start in the low half, length in

@@ -71,8 +71,6 @@ __device__ __forceinline__ uint32_t slot24(int key) {
     return (x >> (24 - kBits)) & (T - 1);
 }
 
-// Whether a matrix has columns that slot24 does not tell apart.
-__device__ __forceinline__ bool far_columns(int columns) { return columns > 1 << 24; }
 template <int T, bool FAR>
 __device__ __forceinline__ uint32_t walk_slot(int key) {
     if constexpr (FAR)
@@ -134,9 +132,9 @@ struct SlotWord {
     static constexpr int kBits = __builtin_ctz(T);
     int shift;       // scalar: kBits or 0
     uint32_t slots;  // scalar: T - 1 or 0
-    bool far;        // scalar: far_columns
+    bool far;        // scalar: more than 2^24 columns
     __device__ __forceinline__ explicit SlotWord(int columns)
-        : shift(columns < (1 << (32 - kBits)) ? kBits : 0), slots(shift ? T - 1 : 0), far(far_columns(columns)) {}
+        : shift(columns < (1 << (32 - kBits)) ? kBits : 0), slots(shift ? T - 1 : 0), far(columns > 1 << 24) {}
     __device__ __forceinline__ uint32_t pack(int key, int slot) const {
         return static_cast<uint32_t>(key) << shift | (static_cast<uint32_t>(slot) & slots);
     }
@@ -367,13 +365,13 @@ struct WaveOperands {
     const long long SPG_GLOBAL* bref;
     const int32_t SPG_GLOBAL* b_col;
     const V SPG_GLOBAL* b_val;
-    bool wide;  // B's arrays may pass 4 GiB: 64-bit offsets
-    bool far;   // far_columns of B
+    int wide;  // WideFlags
 };
 
 // The products of A's entries [a0, a1), in rounds of N * 64:
 // f(key[N], prod[N], ok[N], far), ok[j] the lanes with a product j, far the
-// constant FAR (far_columns of B).  The wave takes 64 entries at a time, one to a
+// constant WIDE (B has one of the WideFlags: 64-bit offsets and a 32-bit
+// hash).  The wave takes 64 entries at a time, one to a
 // lane; entries with an empty row of B drop out.  A product's entry is the
 // number of entries that start at or before it (less one): the chunk's
 // starts are marked in a bitmap, 64 products to a word and one position
@@ -383,7 +381,7 @@ struct WaveOperands {
 // ... of the row, counted on over its windows and chunks, or, with `by_chunk`,
 // every round of the chunks first, first + step, ... instead.  An f that
 // returns false (the same on every lane) ends the walk.
-template <typename V, int N, bool VALS, bool WIDE, bool FAR, typename F>
+template <typename V, int N, bool VALS, bool SHARED, bool WIDE, typename F>
 __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
                                                  int first, int step, bool by_chunk) {
     static_assert(N <= kWavePad, "a round may pass the window by N - 1 words");
@@ -413,9 +411,13 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
         for (int win = 0; win < total; win += kWave * kWaveWords) {
             const int in_win = min(total - win, kWave * kWaveWords);
             const int n_rounds = (in_win + N * kWave - 1) / (N * kWave);
-            if (r >= n_rounds) {  // the other waves' rounds
-                r -= n_rounds;
-                continue;
+            if constexpr (SHARED) {
+                if (r >= n_rounds) {  // the other waves' rounds
+                    r -= n_rounds;
+                    continue;
+                }
+            } else {
+                r = 0;
             }
             wave_sync();  // the previous window's reads are done
             if (lane < kWaveWords + kWavePad) wc->starts[lane] = 0;
@@ -474,7 +476,7 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
 #pragma unroll
                     for (int j = 0; j < N; ++j) prod[j] = a[j] * static_cast<LdsSum>(bv[j]);
                 }
-                constexpr std::bool_constant<FAR> far{};
+                constexpr std::bool_constant<WIDE> far{};
                 if constexpr (std::is_same_v<decltype(f(key, prod, ok, far)), bool>) {
                     if (!f(key, prod, ok, far)) return;
                 } else {
@@ -486,16 +488,26 @@ __device__ __forceinline__ void wave_products_at(const WaveOperands<V>& W, int a
     }
 }
 
+template <typename V, int N, bool VALS, bool SHARED, typename F>
+__device__ __forceinline__ void wave_products_shared(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
+                                                     int first, int step, bool by_chunk) {
+    // Two copies of the walk: choosing the hash round by round cost the 96^3 stencil 5 %, a third copy for wide
+    // columns at narrow offsets 1.6 %.
+    if (W.wide)
+        wave_products_at<V, N, VALS, SHARED, true>(W, a0, a1, wc, f, first, step, by_chunk);
+    else
+        wave_products_at<V, N, VALS, SHARED, false>(W, a0, a1, wc, f, first, step, by_chunk);
+}
+// A row of this wave alone.
+template <typename V, int N, bool VALS, typename F>
+__device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f) {
+    wave_products_shared<V, N, VALS, false>(W, a0, a1, wc, f, 0, 1, true);
+}
+// This wave's share of a row.
 template <typename V, int N, bool VALS, typename F>
 __device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, int a1, WaveChunk<VALS>* wc, F&& f,
-                                              int first = 0, int step = 1, bool by_chunk = true) {
-    // (a copy of the walk each: chosen round by round instead, the hash cost the 96^3 stencil 5 %)
-    if (W.wide)
-        wave_products_at<V, N, VALS, true, true>(W, a0, a1, wc, f, first, step, by_chunk);
-    else if (W.far)
-        wave_products_at<V, N, VALS, false, true>(W, a0, a1, wc, f, first, step, by_chunk);
-    else
-        wave_products_at<V, N, VALS, false, false>(W, a0, a1, wc, f, first, step, by_chunk);
+                                              int first, int step, bool by_chunk) {
+    wave_products_shared<V, N, VALS, true>(W, a0, a1, wc, f, first, step, by_chunk);
 }
 
 // How the waves of a workgroup share a row: by chunks of 64 entries, or by
@@ -504,12 +516,17 @@ __device__ __forceinline__ void wave_products(const WaveOperands<V>& W, int a0, 
 // the busiest wave's share of them, with their rounds, is the shorter.
 template <int WAVES>
 __device__ __forceinline__ bool wave_by_chunk(int entries, int nip) {
-    constexpr int kRead = 2;  // rounds that take as long as reading a chunk
+    constexpr unsigned kRead = 2;  // rounds that take as long as reading a chunk
+    // Four waves, of which a launch has many rows, do with less (the sum below took the count of 81-entry rows 1.5 %
+    // longer): the two meet at four rounds a chunk with two chunks and about sixteen with four to seven, and the way
+    // picked so is at most 1.43 times as long as the other (three chunks of five rounds).
+    if constexpr (WAVES <= 4)
+        return entries >= 2 * WAVES * kWave || (entries > kWave && nip >> (entries > 3 * kWave ? 6 : 4) <= entries);
     if (entries <= kWave) return false;
     if (entries >= 8 * WAVES * kWave) return true;
-    const int chunks = (entries + kWave - 1) / kWave;
-    const int share = (chunks + WAVES - 1) / WAVES;
-    const int rounds = nip / (4 * kWave) + chunks;
+    const unsigned chunks = static_cast<unsigned>(entries + kWave - 1) / kWave;
+    const unsigned share = (chunks + WAVES - 1) / WAVES;
+    const unsigned rounds = static_cast<unsigned>(nip) / (4 * kWave) + chunks;
     // share * (kRead + rounds / chunks) < kRead * chunks + rounds / WAVES
     return rounds * (share * WAVES - chunks) < kRead * WAVES * chunks * (chunks - share);
 }

@@ -19,7 +19,7 @@ template <int WAVES>
 void k_share(const long long* bref, const int32_t* b_col, int entries, bool by_chunk, int* rounds, int* hits) {
     __shared__ WaveChunk<false> walk[WAVES];
     const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
-    const WaveOperands<double> W{nullptr, bref, b_col, nullptr, false, false};
+    const WaveOperands<double> W{nullptr, bref, b_col, nullptr, 0};
     wave_products<double, kN, false>(
         W, 0, entries, &walk[wave],
         [&](const int(&key)[kN], const LdsSum(&)[kN], const unsigned long long(&ok)[kN], auto) {
