@@ -588,7 +588,7 @@ spg_status ensure_context(Context*& out) {
     c.clock_khz = prop.clockRate;
     c.global_mem = prop.totalGlobalMem;
     if (c.lds < kNumBigLds + 1024 ||
-        c.lds < 4 * sym_row_ints(kSymVariants[kSymMaxVariant]) + 1024)
+        c.lds < kSymMaxLds + 1024)
         return fail(SPG_ERR_UNSUPPORTED_DEVICE, "device offers less LDS per workgroup than the kernels need");
     SPG_TRY(lane_create(c.lane));
     SPG_TRY(lane_create(c.noalloc_lane));

@@ -99,26 +99,39 @@ __device__ __forceinline__ void sym_wave_rows(const ProbSet<V>& ps, const int2* 
     }
 }
 
-// A row of a whole workgroup: every wave walks a share of the products on
-// its own (no barrier inside the walk), all insert into one table.  LIMIT >
-// 0: a wave stops inserting once the row has more than LIMIT distinct
-// columns; returns the count (above LIMIT: too many), the same on every lane.
-template <typename V, int WG, int T, int N, int LIMIT>
-__device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* smem) {
+// A row of WG threads (tid: the thread's place among them), a whole workgroup
+// or an equal share of one whose shares all call this together: every wave
+// walks a share of the products on its own (no barrier inside the walk), all
+// insert into one table.  SHARE: a share, whose row may be -1, none.  LIMIT > 0: a wave stops inserting
+// once the row has more than LIMIT distinct columns; with GUESS also once
+// 15/16 of the first four rounds' products or more were new columns and so
+// many products promise more than LIMIT.  Returns the count (above LIMIT: too
+// many, or so it seems), the same on every lane.
+template <typename V, int WG, int T, int N, int LIMIT, bool GUESS = false, bool SHARE = false>
+__device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* smem, int tid) {
     typedef int Words __attribute__((vector_size(16)));
     constexpr int kWaves = WG / kWave;
     static_assert(T % (4 * WG) == 0, "every thread clears a whole share");
-    const int wave = uniform(static_cast<int>(threadIdx.x) / kWave);
+    const int wave = uniform(tid / kWave);
     int* tab = smem;
     auto* walk = reinterpret_cast<WaveChunk<false>*>(smem + T);
     int* total = reinterpret_cast<int*>(walk + kWaves);
 #pragma unroll
     for (int i = 0; i < T / (4 * WG); ++i)
-        reinterpret_cast<Words*>(tab)[i * WG + threadIdx.x] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
-    if (threadIdx.x == 0) *total = 0;
+        reinterpret_cast<Words*>(tab)[i * WG + tid] = Words{kEmpty, kEmpty, kEmpty, kEmpty};
+    if (tid == 0) *total = 0;
     const WaveOperands<V> W{nullptr, uniform_ptr(P.bref), uniform_ptr(P.b_col), nullptr, uniform(P.wide)};
-    const int a0 = uniform(P.a_rpt[row]), a1 = uniform(P.a_rpt[row + 1]);
-    const int nip = uniform(P.nip[row]);
+    int a0 = 0, a1 = 0, nip = 0;
+    if (!SHARE || row >= 0) {
+        a0 = uniform(P.a_rpt[row]);
+        a1 = uniform(P.a_rpt[row + 1]);
+        nip = uniform(P.nip[row]);
+    }
+    // GUESS: `total` holds the products so far (modulo 2^18) above the count
+    constexpr int kCountBits = GUESS ? 14 : 31;
+    constexpr unsigned kCount = (1u << kCountBits) - 1;
+    static_assert(!GUESS || LIMIT + N * WG <= static_cast<int>(kCount), "the count's bits");
+    const unsigned sample = nip > LIMIT + LIMIT / 16 ? N * WG : UINT_MAX;
     __syncthreads();
     int added = 0;
     auto report = [&]() {
@@ -130,7 +143,12 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
         [&](const int(&key)[N], const LdsSum(&)[N], const unsigned long long(&ok)[N], auto far) -> bool {
             if constexpr (LIMIT > 0) {
                 const int have = uniform(lds_load(total));
-                if (have > LIMIT) return false;
+                if constexpr (GUESS) {
+                    const unsigned seen = static_cast<unsigned>(have) >> kCountBits, count = have & kCount;
+                    if (count > LIMIT || (seen >= sample && 16 * count >= 15 * seen)) return false;
+                } else {
+                    if (have > LIMIT) return false;
+                }
                 // Near the limit a slot at a time, which leaves the table with LIMIT + 64 columns a wave instead
                 // of LIMIT + 256: with 16 waves 83 % full instead of 92 (500 rows of 40,000 columns stop after
                 // 610 us with whole rounds, after 230 so).
@@ -149,27 +167,64 @@ __device__ __forceinline__ int sym_group_row(const GProb<V>& P, int row, int* sm
             }
             uint32_t h[N];
             table_slots<T, far, N, true>(tab, key, ok, h, added);
+            if constexpr (GUESS) {
+#pragma unroll
+                for (int j = 0; j < N; ++j) added += __popcll(ok[j]) << kCountBits;
+            }
             if constexpr (LIMIT > 0) report();
             return true;
         },
         wave, kWaves, wave_by_chunk<kWaves>(a1 - a0, nip));
     report();
     __syncthreads();
-    const int n = *total;
+    int n = *total;
+    if constexpr (GUESS) {
+        const unsigned missing = (static_cast<unsigned>(n) ^ static_cast<unsigned>(nip) << kCountBits) >> kCountBits;
+        n = missing ? LIMIT + 1 : n & kCount;  // (stopped: not all products)
+    }
     __syncthreads();  // the table and the total are reused by the next row
     return n;
 }
 
-template <int VV>
-constexpr int sym_unit_lds() {
-    return 4 * kSymVariants[VV].r * sym_row_ints(kSymVariants[VV]);
+// Where the rows go that variant 8 hands on to the largest-table launch.
+struct OverLists {
+    int2* items;  // behind the last bin's list: rows of more than kSymSmallNip products
+    int2* last;   // from here down: the others
+};
+
+// One wave hands on rows k, k + step, ... (n <= 64 of them) below end: an
+// atomic for each of the two lists, however many rows it takes (about 10 ns
+// each from all workgroups: 200 us for 20,000 rows one by one).
+template <typename V>
+__device__ __forceinline__ void hand_on(const ProbSet<V>& ps, const int2* __restrict__ bin_items, int k, int step,
+                                        int n, int end, const OverLists& over, DevMeta* meta) {
+    const int lane = lane_id();
+    const bool ok = lane < n && k + lane * static_cast<long long>(step) < end;
+    int2 it = make_int2(0, 0);
+    int nip = 0;
+    if (ok) {
+        it = bin_items[k + lane * step];
+        nip = ps.get(it.x).nip[it.y];
+    }
+    const unsigned long long small = __ballot(ok && nip <= kSymSmallNip), large = __ballot(ok && nip > kSymSmallNip);
+    int at_small = 0, at_large = 0;
+    if (lane == 0) {
+        if (small) at_small = atomicAdd(&meta->fail_count.over_small, __popcll(small));
+        if (large) at_large = atomicAdd(&meta->fail_count.over, __popcll(large));
+    }
+    at_small = uniform(at_small);
+    at_large = uniform(at_large);
+    if (in_mask(small)) over.last[-(at_small + rank_in(small))] = it;
+    if (in_mask(large)) over.items[at_large + rank_in(large)] = it;
 }
 
 // The units k0, k0 + step, ... below k_end (kV.r rows each) of a bin of
-// variant VV.
+// variant VV.  After a row that overflows variant 8's table the workgroup
+// hands its next ones on untried, a few and then more each time (rows of one
+// matrix are alike), until it tries one that fits.
 template <typename V, int VV>
 __device__ __forceinline__ void sym_units(const ProbSet<V>& ps, const int2* __restrict__ bin_items, int k0, int step,
-                                          int k_end, int count, int* smem, int* s_tmp, int2* over_items,
+                                          int k_end, int count, int* smem, int* s_tmp, const OverLists& over,
                                           DevMeta* meta) {
     constexpr SymVariant kV = kSymVariants[VV];
     const int end = min(count, k_end * kV.r);
@@ -179,16 +234,27 @@ __device__ __forceinline__ void sym_units(const ProbSet<V>& ps, const int2* __re
                                         smem + wave * sym_row_ints(kV));
     } else if constexpr (sym_is_group(kV)) {
         constexpr int kLimit = VV == kSymOverVariant ? kSymOverThreshold : 0;
+        // A dozen scalar instructions a round: 59,049 rows of 6,561 products on 375 columns took 458 us instead of
+        // 393 while every row was guessed at.  The first one is, and those after one that overflowed.
+        bool guess = true;
+        int untried = 0;
         for (int k = k0; k < end; k += step) {
             const int2 it = bin_items[k];
             const GProb<V> P = ps.get(uniform(it.x));
             const int row = uniform(it.y);
-            const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kLimit>(P, row, smem);
-            if (threadIdx.x == 0) {
-                if (kLimit > 0 && n > kLimit)
-                    over_items[atomicAdd(&meta->fail_count.over, 1)] = it;
-                else
-                    P.c_rpt[row] = n;
+            const int n = kLimit > 0 && guess
+                              ? sym_group_row<V, kV.wg, kV.t, kV.pmax, kLimit, true>(P, row, smem, threadIdx.x)
+                              : sym_group_row<V, kV.wg, kV.t, kV.pmax, kLimit>(P, row, smem, threadIdx.x);
+            guess = kLimit > 0 && n > kLimit;
+            if (guess) {
+                untried = min(2 * untried + 3, kWave - 1);
+                if (uniform(static_cast<int>(threadIdx.x) / kWave) == 0)
+                    hand_on<V>(ps, bin_items, k, step, untried + 1, end, over, meta);
+                if (end - k <= untried * static_cast<long long>(step)) break;
+                k += untried * step;
+            } else {
+                untried = 0;
+                if (threadIdx.x == 0) P.c_rpt[row] = n;
             }
         }
     } else {
@@ -214,7 +280,8 @@ __global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves) 
     __syncthreads();
     const int xcd = blockIdx.x % kXcds;
     const int step = gridDim.x / kXcds;
-    int2* over_items = items + static_cast<long long>(sym.n - 1) * bin_cap + meta->sym_count[sym.n - 1].v;
+    int2* last_bin = items + static_cast<long long>(sym.n - 1) * bin_cap;
+    const OverLists over{last_bin + meta->sym_count[sym.n - 1].v, last_bin + bin_cap - 1};
     int k0 = blockIdx.x / kXcds;  // this workgroup's first unit in the XCD's slice of the bin
     for (int b = n_multi - 1; b >= 0; --b) {
         const int count = s_cnt[b];
@@ -227,7 +294,7 @@ __global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves) 
         const int first = xcd * per;
 #define SPG_SYM_CASE(v)                                                                                            \
     case v:                                                                                                        \
-        sym_units<V, v>(ps, bin_items, first + k0, step, first + per, count, smem, s_tmp, over_items, meta);       \
+        sym_units<V, v>(ps, bin_items, first + k0, step, first + per, count, smem, s_tmp, over, meta);             \
         break;
         switch (sym.variant[b]) {
             SPG_SYM_CASE(0)
@@ -255,20 +322,25 @@ __global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves) 
 // Largest LDS table (32768 slots, 128 KiB) with overflow detection
 // (sym1.cuh:169-245): a row whose distinct count passes 80 % of the table
 // stops early and is queued, with its global-table slot range, for
-// k_sym_global.
+// k_sym_global.  Then, where they are many, the rows handed on that cannot
+// fill a table of 8192, four at a time with a quarter of the workgroup each: one
+// by one they took 304 us for 20,000 rows of 2,304 products, so 175 us.
 template <typename V>
 __global__ __launch_bounds__(1024) void k_sym_max(ProbSet<V> ps, const int2* __restrict__ items, int bin_cap,
                                                   int bin, DevMeta* __restrict__ meta,
                                                   int2* __restrict__ fail_items, long long* __restrict__ fail_off) {
     constexpr SymVariant kV = kSymVariants[kSymMaxVariant];
-    __shared__ __align__(16) int smem[sym_unit_lds<kSymMaxVariant>() / 4];
+    __shared__ __align__(16) int smem[kSymMaxLds / 4];
     const int2* bin_items = items + static_cast<long long>(bin) * bin_cap;
-    const int count = meta->sym_count[bin].v + meta->fail_count.over;
+    const int large = meta->sym_count[bin].v + meta->fail_count.over;
+    const int small = meta->fail_count.over_small;
+    const bool shares = small > static_cast<int>(gridDim.x);  // (fewer have a workgroup each)
+    const int count = large + (shares ? 0 : small);
     for (int u = blockIdx.x; u < count; u += gridDim.x) {
-        const int2 it = bin_items[u];
+        const int2 it = bin_items[u < large ? u : bin_cap - 1 - (u - large)];
         const GProb<V> P = ps.get(uniform(it.x));
         const int row = uniform(it.y);
-        const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kSymMaxThreshold>(P, row, smem);
+        const int n = sym_group_row<V, kV.wg, kV.t, kV.pmax, kSymMaxThreshold>(P, row, smem, threadIdx.x);
         if (threadIdx.x == 0) {
             if (n <= kSymMaxThreshold) {
                 P.c_rpt[row] = n;
@@ -279,6 +351,20 @@ __global__ __launch_bounds__(1024) void k_sym_max(ProbSet<V> ps, const int2* __r
                     atomicAdd(&meta->fail_pool.v, static_cast<unsigned long long>(global_table_slots(P.nip[row]))));
             }
         }
+    }
+    constexpr int kShares = kV.wg / kSymSmall.wg;
+    static_assert(kShares * sym_row_ints(kSymSmall) * 4 <= kSymMaxLds && sym_row_ints(kSymSmall) % 4 == 0,
+                  "a share's LDS");
+    if (!shares) return;
+    const int share = uniform(static_cast<int>(threadIdx.x) / kSymSmall.wg);
+    for (int u = blockIdx.x * kShares; u < small; u += gridDim.x * kShares) {
+        const bool mine = u + share < small;
+        const int2 it = bin_items[bin_cap - 1 - (mine ? u + share : u)];
+        const GProb<V> P = ps.get(uniform(it.x));
+        const int row = mine ? uniform(it.y) : -1;
+        const int n = sym_group_row<V, kSymSmall.wg, kSymSmall.t, kSymSmall.pmax, 0, false, true>(
+            P, row, smem + share * sym_row_ints(kSymSmall), threadIdx.x % kSymSmall.wg);
+        if (mine && threadIdx.x % kSymSmall.wg == 0) P.c_rpt[row] = n;
     }
 }
 

@@ -195,12 +195,14 @@ struct alignas(128) Counter {
     T v;
 };
 
-// Rows that moved on during the count: `v` overflowed the largest table,
-// `over` were added to the last bin's list by its overflowing neighbour (both
-// rare, so they share a line).
+// Rows that moved on during the count: `v` overflowed the largest table;
+// `over` and `over_small` were handed to the largest-table launch by its
+// neighbour, behind the last bin's list and from the end of its region down
+// (all updated a few times a workgroup at most, so they share a line).
 struct alignas(128) RowLists {
     int32_t v;
     int32_t over;
+    int32_t over_small;
 };
 
 // Device counters of one multiply (zeroed by k_clear, or by the read-back

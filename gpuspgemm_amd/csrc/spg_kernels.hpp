@@ -53,6 +53,11 @@ constexpr int kSymOverThreshold = 2048;  // 50 % of 4096
 constexpr int kSymMaxThreshold = 26214;  // 80 % of 32768
 static_assert(kSymOverThreshold + 4 * 256 < 4096 && kSymMaxThreshold + 16 * 256 < 32768,
               "a counting table keeps room for the rounds in flight");
+// Rows that variant 8 hands on and that have at most kSymSmallNip products are
+// counted by the largest-table launch four at a time, in tables of twice
+// their products.
+constexpr int kSymSmallNip = 4096;
+constexpr SymVariant kSymSmall = {256, 1, 2 * kSymSmallNip, 64, 4};
 constexpr int kSymMultiLds = 23 * 1024;  // bytes a workgroup of the multi-bin launch may use (seven on a CU)
 constexpr int kSymMultiMinWaves = 7;     // waves per SIMD it keeps: at most 72 VGPRs
 constexpr bool sym_is_wave(const SymVariant& v) { return v.wg / v.r == kWave; }
@@ -144,6 +149,9 @@ constexpr int sym_row_ints(const SymVariant& v) {
     if (sym_is_wave(v)) return v.t + static_cast<int>(sizeof(WaveChunk<false>)) / 4;
     return padded_row_ints(4 * v.t + (v.wg / v.r > 1 ? 8 * v.ec + 8 : 0));
 }
+constexpr int kSymMaxLds = 4 * (sym_row_ints(kSymVariants[kSymMaxVariant]) > 4 * sym_row_ints(kSymSmall)
+                                    ? sym_row_ints(kSymVariants[kSymMaxVariant])
+                                    : 4 * sym_row_ints(kSymSmall));
 constexpr int max_sym_multi_lds() {
     int m = 0;
     for (int i = 0; i < kSymMultiVariants; ++i) {

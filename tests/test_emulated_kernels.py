@@ -534,6 +534,37 @@ def test_symbolic_overflow_moves_to_the_largest_table(emu, tmp_path):
     run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A1, B1, "--f32", tables=table))
 
 
+def test_rows_past_the_counting_table_are_tried_once(emu, tmp_path):
+    """24 rows in the bin whose table takes 2,048 columns, three to an
+    emulated workgroup: 16 of 2,304 products on about 2,180 columns, two of
+    4,800 on about 4,270 and six of 2,400 on 300.  A row that overflows
+    takes the next ones of its workgroup with it to the largest-table
+    launch, whatever they are, where the shorter ones, more than there are
+    workgroups, are counted four at a time.  Every row of C must be right,
+    and few products may be counted twice: 1.4 compare-and-swaps for every
+    one that a count and a fused pass cannot do without (1.3 so; 1.7 when
+    every row was tried until its table was full)."""
+    rng = np.random.default_rng(12)
+    b_rows = [np.sort(rng.choice(20_000, 48, replace=False)) for _ in range(200)]
+    b_rows += [np.sort(rng.choice(300, 48, replace=False)) for _ in range(60)]
+    a_rows = []
+    for i in range(24):
+        if i % 4 == 3:
+            a_rows.append(200 + np.sort(rng.choice(60, 50, replace=False)))
+        else:
+            a_rows.append(np.sort(rng.choice(200, 100 if i in (5, 12) else 48, replace=False)))
+
+    def matrix(rows, n):
+        rpt = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+        col = np.concatenate(rows).astype(np.int32)
+        return HostCSR(len(rows), n, rpt, col, rng.uniform(-1, 1, col.size))
+    A, B = matrix(a_rows, 260), matrix(b_rows, 20_000)
+    out = run_emu(emu, tmp_path, A, B, env={"EMU_COUNT_CAS": "1"})
+    products, nnz = int(oracle.nip_rows(A, B).sum()), int(oracle.spgemm(A, B).nnz)
+    cas = int(out.split("compare-and-swaps ")[1].split()[0])
+    assert cas <= 1.4 * (products + nnz), (cas, products, nnz)
+
+
 def test_global_paths(emu, tmp_path):
     """The heavy-row case first with the default tables, a long row of the
     largest LDS variants, and then with every row forced to the global
