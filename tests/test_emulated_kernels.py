@@ -398,6 +398,24 @@ def test_sorted_rows(emu, tmp_path, variant, products, columns):
     run_emu_all(emu, tmp_path, call(A, B, tables=table), call(A, B, "--f32", tables=table))
 
 
+@pytest.mark.parametrize("b", [5, 6, 8])
+def test_many_products_on_few_columns(emu, tmp_path, b):
+    """Dense blocks of b rows: b * b products on b columns.  The default
+    tables give such rows to a variant with few lanes to a row (one that
+    sorts them needs a lane for each product)."""
+    m = 12 * b
+    i = np.arange(m)
+    col = (i // b * b)[:, None] + np.arange(b)[None, :]
+    A = HostCSR(m, m, (np.arange(m + 1) * b).astype(np.int32), col.ravel().astype(np.int32),
+                np.random.default_rng(b).uniform(-1, 1, m * b))
+    out = run_emu(emu, tmp_path, A, A, env={"SPG_LOG_LEVEL": "debug"})
+    fused = next(x for x in out.splitlines() if "fused bins: " in x).split("fused bins: ")[1].split(", ")
+    line = next(x for x in out.splitlines() if "symbolic phase" in x)
+    rows = [int(x) for x in line.split("rows per fused bin [")[1].split("]")[0].split()]
+    taken = [int(fused[k].split()[0][1:]) for k in range(len(rows)) if rows[k]]
+    assert sum(rows) == m and [NUM[v][0] for v in taken] == [8], (taken, rows)
+
+
 @pytest.mark.parametrize("variant", [v["id"] for v in _NV if not v["global"] and v["lanes"] == 256 and v["chunk"] == 64])
 def test_group_rows_and_column_counts(emu, tmp_path, variant):
     """Rows that the waves of a workgroup share, filled to one short of the
