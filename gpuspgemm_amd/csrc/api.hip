@@ -61,6 +61,10 @@ static __device__ __align__(256) char scratch[kNoAllocScratch];
 // 2048 tiles, 2 * 10^9 at 2^27 rows).
 constexpr int kTilePrefixMin = 2048;
 
+// Entries of B that 32-bit byte offsets reach in any case: 2^29 values of 8
+// bytes are 4 GiB.
+constexpr int kWideMinMax = 1 << 29;
+
 thread_local std::string g_last_error;
 
 spg_status fail(spg_status s, const std::string& msg) {
@@ -466,8 +470,8 @@ struct Context {
     // in the tile count); SPG_TILE_PREFIX_MIN overrides it
     int tile_prefix_min = kTilePrefixMin;
     // entries of B from which the kernels take 64-bit byte offsets into its
-    // arrays (8 bytes a value pass 4 GiB there); SPG_WIDE_MIN overrides it
-    int wide_min = 1 << 29;
+    // arrays (8 bytes a value pass 4 GiB there); SPG_WIDE_MIN lowers it
+    int wide_min = kWideMinMax;
     Lane lane;  // graph replay and profiling run here, one call at a time
     Lane noalloc_lane;             // spg_multiply_noalloc, one call at a time
     char* noalloc_base = nullptr;  // this device's address of `scratch`
@@ -600,13 +604,14 @@ spg_status ensure_context(Context*& out) {
     c.occ_sym_multi = std::min(occupancy_sym_multi<double>(), occupancy_sym_multi<float>());
     c.occ_sym_max = occupancy_sym_max<double>();
     if (const char* env = std::getenv("SPG_TILE_PREFIX_MIN")) c.tile_prefix_min = std::max(1, std::atoi(env));
-    if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::max(0, std::atoi(env));
+    if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::min(kWideMinMax, std::max(0, std::atoi(env)));
     for (int v = 0; v < kNumVariantCount; ++v) {
         c.occ_num[0][v] = occupancy_symnum_bin<float>(v);
         c.occ_num[1][v] = occupancy_symnum_bin<double>(v);
     }
-    log_msg(kDebug, "context on device %d (%s, %d CUs); symbolic bins: %s; fused bins: %s", dev, c.arch.c_str(),
-            c.cus, table_text(c.sym).c_str(), table_text(c.num).c_str());
+    log_msg(kDebug,
+            "context on device %d (%s, %d CUs); 64-bit offsets from %d entries of B; symbolic bins: %s; fused bins: %s",
+            dev, c.arch.c_str(), c.cus, c.wide_min, table_text(c.sym).c_str(), table_text(c.num).c_str());
     c.ready.store(true, std::memory_order_release);
     return SPG_OK;
 }

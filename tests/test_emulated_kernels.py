@@ -363,6 +363,15 @@ def test_wave_rows_windows_and_wide_offsets(emu, tmp_path, variant):
                 call(A.astype(np.float32), B.astype(np.float32), "--f32", tables=table, env={"SPG_WIDE_MIN": "0"}))
 
 
+def test_wide_offsets_start_where_narrow_ones_end(emu, tmp_path):
+    """SPG_WIDE_MIN cannot be raised past the 2^29 entries whose values
+    32-bit byte offsets reach."""
+    A = gen.uniform8(m=64, per_row=2, seed=3, n=64)
+    for value, used in (("2147483647", 1 << 29), (str((1 << 29) + 1), 1 << 29), ("1000", 1000), ("-5", 0)):
+        out = run_emu(emu, tmp_path, A, A, env={"SPG_WIDE_MIN": value, "SPG_LOG_LEVEL": "debug"})
+        assert f"64-bit offsets from {used} entries of B" in out, out
+
+
 # fused variants that sort rows of at most `products` in registers
 SORTED = [(v, NUM[v][2]) for v in sorted(NUM) if NUM[v][0] == NUM[v][2] or (NUM[v][0] == 64 and NUM[v][2] <= 128)]
 
