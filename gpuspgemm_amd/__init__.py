@@ -124,13 +124,16 @@ def get_variants(phase: int) -> str:
 def variant_list(phase: int) -> list[dict]:
     """Compiled kernel variants of a phase as dicts: id, wg, rows, lanes
     (per row), table (phase 0) or capacity (phase 1), chunk, slots, and the
-    flags max (phase 0's overflow-detecting variant) / global (phase 1's
-    global-memory variant), and merged: the merged launch set (0 small
-    rows, 1 longer rows) whose bins share one launch, or None."""
+    flags max (phase 0's largest table) / over (phase 0: takes rows of any
+    NIP and hands on those that fill its table) / global (phase 1's
+    global-memory variant) / staged (phase 1: walks a row once only if its
+    products fit lanes * slots; the others walk once whatever the NIP), and
+    merged: the merged launch set (0 small rows, 1 longer rows) whose bins
+    share one launch, or None."""
     out = []
     for line in get_variants(phase).splitlines():
         parts = line.split()
-        v = {"id": int(parts[0]), "max": "max" in parts[1:], "global": "global" in parts[1:], "merged": None}
+        v = {"id": int(parts[0]), "merged": None, **{k: k in parts[1:] for k in ("max", "over", "global", "staged")}}
         for kv in parts[1:]:
             if "=" in kv:
                 k, x = kv.split("=")

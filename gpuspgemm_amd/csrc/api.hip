@@ -1920,12 +1920,15 @@ spg_status spg_get_variants(int32_t phase, char* buf, size_t buf_len) {
         for (int v = 0; v <= kSymMaxVariant; ++v)
             out << v << " wg=" << kSymVariants[v].wg << " rows=" << kSymVariants[v].r << " table=" << kSymVariants[v].t
                 << " chunk=" << kSymVariants[v].ec << " slots=" << kSymVariants[v].pmax
-                << (v == kSymMaxVariant ? " max" : "") << '\n';
+                << (v == kSymMaxVariant ? " max" : "") << (v == kSymOverVariant ? " over" : "") << '\n';
     } else if (phase == 1) {
         for (int v = 0; v < kNumVariantCount; ++v) {
             if (v == kNumGlobalVariant) continue;
             out << v << " wg=" << kNumVariants[v].wg << " rows=" << kNumVariants[v].r << " capacity="
                 << kNumVariants[v].p << " chunk=" << kNumVariants[v].ec << " slots=" << kNumVariants[v].pmax
+                << (num_is_wave(kNumVariants[v]) || num_is_group(kNumVariants[v]) || num_is_long(kNumVariants[v])
+                        ? ""
+                        : " staged")
                 << (num_multi_set(v) >= 0 ? " merged=" + std::to_string(num_multi_set(v)) : std::string()) << '\n';
         }
         out << kNumGlobalVariant << " global\n";

@@ -9,7 +9,7 @@ by measurement on the GPU it runs on:
 
   * each bin of the default tables is a slot with caps (NIP, nnz); every
     compiled variant whose table / capacity fits the slot's caps is a
-    candidate for it;
+    candidate for it (sym_candidates, num_candidates);
   * slots are tuned one at a time, greedily, in two passes: each candidate
     replaces the slot's variant, or moves one of the slot's caps (halved or
     doubled, where the variant still admits it), and the whole multiply is
@@ -46,23 +46,27 @@ def table_text(rows: list[tuple[int, int, int]]) -> str:
 
 
 def sym_candidates(slot: tuple[int, int, int], variants: list[dict]) -> list[int]:
-    """Multi-bin symbolic variants whose table holds the slot's NIP cap at
-    most half full and is at most 16x larger."""
+    """Multi-bin symbolic variants whose table the slot's NIP cap fills to
+    three quarters at most and that is at most 16x larger, and the variant
+    that takes rows of any NIP for slots that fill half of its table or
+    more."""
     _, nip_cap, _ = slot
     return [v["id"] for v in variants
-            if not v["max"] and 2 * nip_cap <= v["table"] <= 16 * nip_cap]
+            if not v["max"] and (2 * nip_cap >= v["table"] if v["over"]
+                                 else 4 * nip_cap <= 3 * v["table"] <= 48 * nip_cap)]
 
 
 def num_candidates(slot: tuple[int, int, int], variants: list[dict]) -> list[int]:
     """Fused LDS variants whose capacity admits the slot's nnz cap and is at
-    most 8x larger; for a slot whose NIP cap is finite, only variants whose
-    lanes can stage that many products in registers."""
+    most 8x larger; of those that stage products in registers, for a slot
+    whose NIP cap is finite, only variants whose lanes stage at least half
+    as many (the others have no such limit)."""
     _, nip_cap, nnz_cap = slot
     out = []
     for v in variants:
         if v["global"] or not (nnz_cap <= v["capacity"] <= 8 * nnz_cap):
             continue
-        if nip_cap != INT_MAX and v["lanes"] * v["slots"] < nip_cap:
+        if v["staged"] and nip_cap != INT_MAX and 2 * v["lanes"] * v["slots"] < nip_cap:
             continue
         out.append(v["id"])
     return out
@@ -106,7 +110,7 @@ def cap_moves(phase: int, slot: tuple[int, int, int], variants: list[dict]) -> l
     info = next(x for x in variants if x["id"] == v)
     if phase == 0:
         for c in (nip // 2, nip * 2):
-            if 1 <= c < info["table"] and c != nip:
+            if 1 <= c < INT_MAX and (info["over"] or c < info["table"]) and c != nip:
                 out.append((v, c, nnz))
     else:
         if nip != INT_MAX:

@@ -93,6 +93,28 @@ def test_tuner_emits_tables_the_library_accepts(on_emu, tmp_path):
     assert res["sym"][-1][1:] == (INT_MAX, INT_MAX) and res["num"][-1][1:] == (INT_MAX, INT_MAX)
 
 
+def test_default_slots_are_candidates_of_themselves(on_emu):
+    """The tuner times what the library ships: every default bin's variant
+    is among the bin's candidates, with others beside it wherever another
+    variant admits the bin's rows, and the bin whose rows may have any NIP
+    has caps to move to."""
+    sv, nv = g.variant_list(0), g.variant_list(1)
+    for phase, candidates, variants in ((0, tune.sym_candidates, sv), (1, tune.num_candidates, nv)):
+        for slot in tune.parse_table(g.get_tuning(phase))[:-1]:  # (the last bin is fixed)
+            found = candidates(slot, variants)
+            assert slot[0] in found, (phase, slot, found)
+            for v in found:  # and the library admits each of them
+                table = tune.parse_table(g.get_tuning(phase))
+                table[table.index(slot)] = (v, slot[1], slot[2])
+                g.set_tuning(phase, tune.table_text(table))
+                g.set_tuning(phase, None)
+    wave = next(s for s in tune.parse_table(g.get_tuning(1)) if next(
+        v for v in nv if v["id"] == s[0])["lanes"] == 64)
+    assert len(tune.num_candidates(wave, nv)) > 1
+    over = next(s for s in tune.parse_table(g.get_tuning(0)) if next(v for v in sv if v["id"] == s[0])["over"])
+    assert [c for _, c, _ in tune.cap_moves(0, over, sv)] == [over[1] // 2, 2 * over[1]]
+
+
 def test_library_refuses_tables_that_break_the_rules(on_emu):
     sv, nv = g.variant_list(0), g.variant_list(1)
     sym = tune.parse_table(g.get_tuning(0))
