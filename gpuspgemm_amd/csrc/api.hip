@@ -464,7 +464,6 @@ struct Context {
     BinTable sym{};
     BinTable num{};
     int occ_sym_multi = 1, occ_sym_max = 1;
-    int occ_num[2][kNumVariantCount] = {};
     // tiles from which the scan reads each tile's prefix off one scanned
     // array instead of summing the earlier tiles per workgroup (quadratic
     // in the tile count); SPG_TILE_PREFIX_MIN overrides it
@@ -591,8 +590,7 @@ spg_status ensure_context(Context*& out) {
     c.lds = static_cast<int>(prop.sharedMemPerBlock);
     c.clock_khz = prop.clockRate;
     c.global_mem = prop.totalGlobalMem;
-    if (c.lds < kNumBigLds + 1024 ||
-        c.lds < kSymMaxLds + 1024)
+    if (c.lds < kNumBigLds + 1024 || c.lds < kSymMaxLds + 1024)
         return fail(SPG_ERR_UNSUPPORTED_DEVICE, "device offers less LDS per workgroup than the kernels need");
     SPG_TRY(lane_create(c.lane));
     SPG_TRY(lane_create(c.noalloc_lane));
@@ -603,12 +601,10 @@ spg_status ensure_context(Context*& out) {
     SPG_TRY(check_num_table(c.num));
     c.occ_sym_multi = std::min(occupancy_sym_multi<double>(), occupancy_sym_multi<float>());
     c.occ_sym_max = occupancy_sym_max<double>();
+    load_symnum<float>();
+    load_symnum<double>();
     if (const char* env = std::getenv("SPG_TILE_PREFIX_MIN")) c.tile_prefix_min = std::max(1, std::atoi(env));
     if (const char* env = std::getenv("SPG_WIDE_MIN")) c.wide_min = std::min(kWideMinMax, std::max(0, std::atoi(env)));
-    for (int v = 0; v < kNumVariantCount; ++v) {
-        c.occ_num[0][v] = occupancy_symnum_bin<float>(v);
-        c.occ_num[1][v] = occupancy_symnum_bin<double>(v);
-    }
     log_msg(kDebug,
             "context on device %d (%s, %d CUs); 64-bit offsets from %d entries of B; symbolic bins: %s; fused bins: %s",
             dev, c.arch.c_str(), c.cus, c.wide_min, table_text(c.sym).c_str(), table_text(c.num).c_str());

@@ -16,7 +16,7 @@ __device__ __forceinline__ void sym_rows(const ProbSet<V>& ps, const int2* __res
                                          int end, int* smem, int* s_tmp) {
     constexpr int L = WG / R;
     static_assert(WG % R == 0, "bad variant shape");
-    static_assert(L <= kWave || R == 1, "a row spans several waves only when it owns the workgroup");
+    static_assert(L < kWave, "longer rows: sym_wave_rows, sym_group_row");
     using Meta = ChunkMeta<V, EC, false>;
     constexpr int ROW_INTS = sym_row_ints(SymVariant{WG, R, T, EC, PMAX});
     const int slot = threadIdx.x / L;
@@ -39,14 +39,7 @@ __device__ __forceinline__ void sym_rows(const ProbSet<V>& ps, const int2* __res
     for_each_round<V, L, EC, PMAX, false>(
         P, a0, a1, lr, cm, s_tmp,
         [&](const int(&key)[PMAX], const V(&)[PMAX], const bool(&ok)[PMAX]) { mine += table_insert_all<T>(tab, key, ok); });
-    int nnz;
-    if constexpr (L <= kWave) {
-        nnz = group_sum<L>(mine);
-    } else {
-        int total;
-        (void)group_excl_scan<L>(mine, lr, s_tmp, total);
-        nnz = total;
-    }
+    const int nnz = group_sum<L>(mine);
     if (active && lr == 0) P.c_rpt[it.y] = nnz;
     gsync<L>();  // the table is reused by the next unit
 }
@@ -267,8 +260,8 @@ __device__ __forceinline__ void sym_units(const ProbSet<V>& ps, const int2* __re
 // are read on the device, so the launch needs no host round trip; the grid
 // is persistent.  Every XCD takes a contiguous slice of every bin, the bins
 // of long rows first, and its workgroups deal the slices' units among
-// themselves.  One kernel for all variants (72 VGPRs and 23 KB of LDS, seven
-// waves per SIMD) keeps the whole symbolic phase on one stream: in three
+// themselves.  One kernel for all variants (72 VGPRs with 52 bytes spilled a
+// lane, 21.6 KB of LDS, seven waves per SIMD) keeps the whole symbolic phase on one stream: in three
 // launches on three streams, the fork cost 7 to 14 us and the join 10 to 58.
 template <typename V>
 __global__ __launch_bounds__(kMultiThreads) SPG_WAVES_PER_EU(kSymMultiMinWaves) void k_sym_multi(

@@ -83,8 +83,11 @@ __device__ __forceinline__ int sort_row(const int* tab, int* cols, int lr, int* 
 // word, the groups sort the words, a slot whose column differs from the one
 // below starts an entry of C, and its place in the row is the number of such
 // slots before it.  No table, no probing, and LDS sums only for waves that
-// have a repeated column.  Bound by VALU issue (about 100 instructions for
-// the 8 rows of a wave at L = 8, where the hashed path spends 25 a row).
+// have a repeated column.  About 100 vector instructions for the 8 rows of a
+// wave at L = 8, where the hashed path spends 25 a row: on the power-law matrix
+// 45 of the launch's 105 us, which is bound by the lines of B that it fetches
+// past L2.  A row to a wave (L = 64) is bound by the instructions of its sort,
+// so rows of few columns are hashed (the bin tables).
 template <int K>
 struct alignas(16) SortSlots {
     unsigned long long starts[K];
@@ -823,15 +826,6 @@ static hipError_t launch_variant(const ProbSet<V>& ps, const RowItem* items, int
     return hipGetLastError();
 }
 
-template <typename V, int VV>
-static int occupancy_variant() {
-    constexpr auto kernel = k_symnum_bin<V, VV>;
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kNumVariants[VV].wg, 0) != hipSuccess) n = 1;
-    return n > 0 ? n : 1;
-}
-
-
 template <typename V>
 hipError_t launch_symnum_bin(int variant, const ProbSet<V>& ps, const RowItem* items, int item_off, int count,
                              DevMeta* meta, int grid, hipStream_t s) {
@@ -867,16 +861,15 @@ void launch_symnum_global(const ProbSet<V>& ps, const RowItem* items, const long
 }
 
 template <typename V>
-int occupancy_symnum_bin(int variant) {
-#define SPG_OCC_CASE(v) \
-    case v:             \
-        return occupancy_variant<V, v>();
-    switch (variant) {
-        SPG_NUM_VARIANTS(SPG_OCC_CASE)
-        default:
-            return 1;
+void load_symnum() {
+    int n = 0;
+#define SPG_LOAD_CASE(v)                                                                                             \
+    {                                                                                                                \
+        constexpr auto kernel = k_symnum_bin<V, v>;                                                                  \
+        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, kNumVariants[v].wg, 0);                       \
     }
-#undef SPG_OCC_CASE
+    SPG_NUM_VARIANTS(SPG_LOAD_CASE)
+#undef SPG_LOAD_CASE
 }
 
 #define SPG_INSTANTIATE_NUM(V)                                                                               \
@@ -886,7 +879,7 @@ int occupancy_symnum_bin(int variant) {
                                                DevMeta*, hipStream_t);                                        \
     template void launch_symnum_global<V>(const ProbSet<V>&, const RowItem*, const long long*, int, int, int*, \
                                           DevMeta*, hipStream_t);                                             \
-    template int occupancy_symnum_bin<V>(int);
+    template void load_symnum<V>();
 
 SPG_INSTANTIATE_NUM(float)
 SPG_INSTANTIATE_NUM(double)

@@ -58,8 +58,8 @@ static_assert(kSymOverThreshold + 4 * 256 < 4096 && kSymMaxThreshold + 16 * 256 
 // their products.
 constexpr int kSymSmallNip = 4096;
 constexpr SymVariant kSymSmall = {256, 1, 2 * kSymSmallNip, 64, 4};
-constexpr int kSymMultiLds = 23 * 1024;  // bytes a workgroup of the multi-bin launch may use (seven on a CU)
-constexpr int kSymMultiMinWaves = 7;     // waves per SIMD it keeps: at most 72 VGPRs
+constexpr int kSymMultiMinWaves = 7;  // waves per SIMD that the multi-bin launch keeps: at most 72 VGPRs
+constexpr int kSymMultiLds = 160 * 1024 / kSymMultiMinWaves;  // bytes a workgroup of it may use: as many on a CU
 constexpr bool sym_is_wave(const SymVariant& v) { return v.wg / v.r == kWave; }
 constexpr bool sym_is_group(const SymVariant& v) { return v.wg / v.r > kWave; }
 
@@ -221,7 +221,7 @@ template <typename V>
 void launch_sym_global(const ProbSet<V>& ps, const int2* fail_items, const long long* fail_off, int* pool,
                        int count, hipStream_t s);
 
-// fused pass: one launch per variant (0..9) over one bin's items
+// fused pass: one launch per variant (all but the global one) over one bin's items
 template <typename V>
 hipError_t launch_symnum_bin(int variant, const ProbSet<V>& ps, const RowItem* items, int item_off, int count,
                              DevMeta* meta, int grid, hipStream_t s);
@@ -234,12 +234,15 @@ template <typename V>
 void launch_symnum_global(const ProbSet<V>& ps, const RowItem* items, const long long* gpool_off, int item_off,
                           int count, int* pool, DevMeta* meta, hipStream_t s);
 
+// has the runtime load the fused kernels (a query of each), for which the first
+// multiply would otherwise wait (5.1 instead of 2.1 ms)
+template <typename V>
+void load_symnum();
+
 // occupancy (workgroups per CU) of the persistent launches
 template <typename V>
 int occupancy_sym_multi();
 template <typename V>
 int occupancy_sym_max();
-template <typename V>
-int occupancy_symnum_bin(int variant);
 
 }  // namespace spg

@@ -9,8 +9,8 @@ from gpuspgemm_amd import timeline
 STEP = [
     ("spg::k_clear(spg::DevMeta*, int)", 1, 0, 1000),
     ("void spg::k_nip<double>(spg::ProbSet<double>, ...)", 1, 1000, 5000),
-    ("void spg::k_sym_multi<double, 0, 4>(...)", 1, 6000, 9000),
-    ("void spg::k_sym_multi<double, 4, 7>(...)", 2, 6500, 8000),
+    ("void spg::k_sym_multi<double>(spg::ProbSet<double>, ...)", 1, 6000, 9000),
+    ("void spg::k_sym_max<double>(spg::ProbSet<double>, ...)", 2, 6500, 8000),
     ("spg::k_total_nip(int const*, ...)", 3, 7000, 30000),  # another call's get_nip: left out
     ("void spg::k_scan_count<double>(...)", 1, 10000, 11000),
     ("spg::k_readback(int const*, ...)", 1, 11000, 12000),
@@ -36,12 +36,13 @@ def test_step_summary(tmp_path):
     steps = timeline.split_multiplies(timeline.load(_trace(tmp_path, [0, 100_000])))
     assert len(steps) == 2
     s = timeline.summarize(steps[0])
-    assert [k["name"] for k in steps[0]][:3] == ["clear", "nip", "sym_multi_small"]
+    assert [k["name"] for k in steps[0]][:3] == ["clear", "nip", "sym_multi"]
+    assert steps[0][3]["name"] == "sym_max"
     assert all(k["name"] != "total_nip" for k in steps[0])
     assert s["span_us"] == 23.0
     # busy: [0, 5] + [6, 9] + [10, 12] + [14, 23] us
     assert s["busy_us"] == 19.0
-    assert [(a, l, b) for a, l, b in s["gaps"]] == [(5.0, 1.0, "sym_multi_small"), (9.0, 1.0, "scan_count"),
+    assert [(a, l, b) for a, l, b in s["gaps"]] == [(5.0, 1.0, "sym_multi"), (9.0, 1.0, "scan_count"),
                                                     (12.0, 2.0, "symnum_v9")]
     assert s["symbolic_us"] == 12.0 and s["readback_to_fused_us"] == 2.0 and s["fused_us"] == 9.0
     assert s["queues"] == {1: (17.0, 7), 2: (9.5, 3)}
