@@ -85,7 +85,7 @@ __device__ __forceinline__ int sort_row(const int* tab, int* cols, int lr, int* 
 // slots before it.  No table, no probing, and LDS sums only for waves that
 // have a repeated column.  About 100 vector instructions for the 8 rows of a
 // wave at L = 8, where the hashed path spends 25 a row: on the power-law matrix
-// 45 of the launch's 105 us, which is bound by the lines of B that it fetches
+// 47 of the launch's 113 us, which is bound by the lines of B that it fetches
 // past L2.  A row to a wave (L = 64) is bound by the instructions of its sort,
 // so rows of few columns are hashed (the bin tables).
 template <int K>
