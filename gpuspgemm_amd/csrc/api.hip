@@ -248,8 +248,12 @@ struct BlockCache {
             Idle& b = it->second;
             if (b.fence && b.fence->ev) {
                 const hipError_t q = hipEventQuery(b.fence->ev);
-                if (q == hipErrorNotReady) continue;
-                if (q != hipSuccess) continue;  // leave it; a later call finds out
+                if (q != hipSuccess) {
+                    // Not ready, or (seen when the thread that recorded the event had ended) an error: leave the
+                    // block, and leave no error behind for the next launch's check to report.
+                    if (q != hipErrorNotReady) (void)hipGetLastError();
+                    continue;
+                }
             }
             *out = b.p;
             live[b.p] = it->first;

@@ -278,7 +278,17 @@ struct hipDeviceProp_t {
 };
 
 inline const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "emulated error"; }
-inline hipError_t hipGetLastError() { return hipSuccess; }
+// the calling thread's last error, as the runtime keeps it (only event
+// queries fail here: EMU_QUERY_ERROR=n fails each thread's n-th)
+inline hipError_t& emu_last_error() {
+    thread_local hipError_t e = hipSuccess;
+    return e;
+}
+inline hipError_t hipGetLastError() {
+    const hipError_t e = emu_last_error();
+    emu_last_error() = hipSuccess;
+    return e;
+}
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipGetDevice(int* d) {
     *d = 0;
@@ -316,7 +326,11 @@ inline hipError_t hipStreamQuery(hipStream_t s) {
     ::emu::drain_stream(s);
     return hipSuccess;
 }
-inline hipError_t hipEventQuery(hipEvent_t e) { return ::emu::event_done(emu_ev(e)) ? hipSuccess : hipErrorNotReady; }
+inline hipError_t hipEventQuery(hipEvent_t e) {
+    thread_local int left = std::getenv("EMU_QUERY_ERROR") ? std::atoi(std::getenv("EMU_QUERY_ERROR")) : 0;
+    if (left > 0 && --left == 0) return emu_last_error() = hipErrorUnknown;
+    return ::emu::event_done(emu_ev(e)) ? hipSuccess : hipErrorNotReady;
+}
 inline hipError_t hipEventSynchronize(hipEvent_t e) {
     ::emu::drain_event(emu_ev(e));
     return hipSuccess;

@@ -631,6 +631,17 @@ def test_noalloc_entry(emu, tmp_path):
     assert out[2].count("structure identical") == 1
 
 
+def test_failed_event_query_is_not_a_failed_multiply(emu, tmp_path):
+    """The block cache asks a released block's event whether its work is
+    done.  A query that fails (seen on the GPU when the thread that had
+    recorded the event was gone) must only pass the block over: the error
+    that it leaves with the runtime must not fail the launches that follow."""
+    A = gen.uniform8(m=64, per_row=4, seed=3, n=64)
+    calls = [call(A, A, "--repeat", "4", env={"EMU_QUERY_ERROR": str(n)}) for n in (1, 2, 3)]
+    for out in run_emu_all(emu, tmp_path, *calls):
+        assert out.count("structure identical") == 4
+
+
 def test_server_batches_and_admission(emu, tmp_path):
     """Served form on the CPU: the same product submitted many times to a
     server with a small maximum batch and a budget of about two outputs,
