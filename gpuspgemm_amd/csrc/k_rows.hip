@@ -307,9 +307,9 @@ __global__ __launch_bounds__(kRowThreads) void k_scan_apply(ProbSet<V> ps, BinTa
         v[j] = r < t.rows ? P.c_rpt[t.row0 + r] : 0;
         nip[j] = r < t.rows ? P.nip[t.row0 + r] : 0;
     }
-    int bin_off = 0;  // thread b < num.n: rows of the bins before b
-    if (threadIdx.x < num.n)
-        for (int b = 0; b < static_cast<int>(threadIdx.x); ++b) bin_off += meta->num_count[b].v;
+    // thread b < num.n: the rows of bin b (a load each side by side: thread b walking the bins before its own took
+    // one after the other, 0.7 us of the launch a bin)
+    const int bin_rows = threadIdx.x < num.n ? meta->num_count[threadIdx.x].v : 0;
 
     // prefix over earlier tiles of this product: read off the scanned tile
     // sums (k_tile_prefix, many tiles), or summed here (few tiles; the
@@ -377,6 +377,13 @@ __global__ __launch_bounds__(kRowThreads) void k_scan_apply(ProbSet<V> ps, BinTa
         if (ps.n_inst == 1) meta->nnz_total.v = run;
     }
     if (flags) atomicOr(&s_flags, flags);
+    int bin_off = bin_rows;  // thread b < num.n: rows of the bins up to b, then of those before b
+#pragma unroll
+    for (int o = 1; o < kMaxBins; o <<= 1) {
+        const int y = __shfl_up(bin_off, o);
+        if (lane_id() >= o) bin_off += y;
+    }
+    bin_off -= bin_rows;
     __syncthreads();
 
     if (threadIdx.x < num.n && s_cnt[threadIdx.x] > 0)
